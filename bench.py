@@ -16,7 +16,7 @@ Reported (one JSON line on stdout):
                int8 Q and the current chunk's ring slot): algorithmic bytes / time, vs 8 TB/s
   cross_attention  the DiT's cross-attention per layer call (6032 queries x 512 context tokens, bf16 MFMA):
                algorithmic flops / time, vs 2.5 PFLOP/s dense bf16
-  fp8_linear   the DiT's FP8 linears at 6032 tokens (rowwise e4m3 activation quant + hipBLASLt FP8 GEMM):
+  fp8_linear   the DiT's FP8 linears at 6032 tokens (rowwise e4m3 activation quant + FP8 GEMM):
                flops / time, vs 5.0 PFLOP/s dense fp8
   chunk_sweep  the whole chunk captured in one HIP graph: 30 layers x 5 passes of the step above, then the
                30-layer re-quant that saves the chunk; seconds per chunk
@@ -418,9 +418,9 @@ DIM, FFN = 1536, 8960       # the DiT's model and feed-forward widths
 
 def fp8_linear_calls(dev, steps=30):
     """The DiT's FP8 linears at the chunk shape (6032 tokens): q/k/v/o (1536 -> 1536) and the two feed-forward
-    layers (1536 -> 8960, 8960 -> 1536). Per call: the activation quantisation (lbw_quant_rows_fp8) and
-    hipBLASLt's rowwise-scaled FP8 GEMM with the bias, timed with hipBLASLt's default solution and with the tuned
-    solution table (`ms` is the latter when the table was read). Flops 2 M K N against 5.0 PFLOP/s dense fp8.
+    layers (1536 -> 8960, 8960 -> 1536), without gradients. Per call: the activation quantisation (lbw_quant_rows_fp8)
+    and the rowwise-scaled FP8 GEMM with the bias (lbw_gemm_fp8_rows; the tuned-solution table of the library GEMM is
+    read for the second timing, `ms`, and changes nothing on this path). Flops 2 M K N against 5.0 PFLOP/s dense fp8.
     act_quant_call_ms times the quantisation call alone from Python; at ~6-9 us of kernel time it is bound by the
     launch path, so it is an upper bound on the kernel."""
     import torch
@@ -431,11 +431,10 @@ def fp8_linear_calls(dev, steps=30):
     stream = torch.cuda.current_stream(dev)
     for name, (k, n) in (("proj_1536x1536", (DIM, DIM)), ("ffn_up_1536x8960", (DIM, FFN)),
                          ("ffn_down_8960x1536", (FFN, DIM))):
-        lin = torch.nn.Linear(k, n).to(torch.bfloat16).to(dev)
+        lin = torch.nn.Linear(k, n).to(torch.bfloat16).to(dev).requires_grad_(False)
         f = FP8Linear(lin)
         x = torch.randn(1, LQ, k, device=dev).to(torch.bfloat16)
         times = {}
-        # hipBLASLt's default solution, then with the tuned-solution table (layers/fp8_gemm_solutions.csv)
         for mode in ("default", "table"):
             table = use_tuned_gemms() if mode == "table" else False
             for _ in range(3):
@@ -453,8 +452,8 @@ def fp8_linear_calls(dev, steps=30):
                      "frac_fp8_peak": round(tf / FP8_PEAK_TFLOPS, 4)}
     # the feed-forward block's GELU + down projection: torch's GELU then the FP8 linear (two passes over the
     # 6032 x 8960 activation), against the GELU fused into the activation quantisation (FP8Linear gelu_input,
-    # what convert_to_fp8(fuse_gelu=True) builds); both with the tuned solution table
-    lin = torch.nn.Linear(FFN, DIM).to(torch.bfloat16).to(dev)
+    # what convert_to_fp8(fuse_gelu=True) builds)
+    lin = torch.nn.Linear(FFN, DIM).to(torch.bfloat16).to(dev).requires_grad_(False)
     plain, fused = FP8Linear(lin), FP8Linear(lin, gelu_input=True)
     h = torch.randn(1, LQ, FFN, device=dev).to(torch.bfloat16)
     table = use_tuned_gemms()
@@ -470,9 +469,9 @@ def fp8_linear_calls(dev, steps=30):
     tunable.enable(False)
     out["ffn_gelu_down_8960x1536"] = {"ms": round(t_fused, 4), "unfused_ms": round(t_unfused, 4),
                                       "gelu_act_quant_call_ms": round(t_gq, 4), "gemm_table": table}
-    # the MXFP8 mode (per-32 E8M0 scales) at the projection shape: its GEMM pads the rows to 128
+    # the MXFP8 mode (per-32 E8M0 scales) at the projection shape
     from lingbot_world_v2_realtime_amd.layers.linear import MXFP8Linear
-    lin = torch.nn.Linear(DIM, DIM).to(torch.bfloat16).to(dev)
+    lin = torch.nn.Linear(DIM, DIM).to(torch.bfloat16).to(dev).requires_grad_(False)
     f = MXFP8Linear(lin)
     x = torch.randn(1, LQ, DIM, device=dev).to(torch.bfloat16)
     for _ in range(3):

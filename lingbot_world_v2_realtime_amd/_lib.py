@@ -1,4 +1,4 @@
-"""ctypes binding of liblbw_attn.so (the C-ABI declared in include/lbw_attn.h)."""
+"""ctypes binding of liblbw_attn.so (the C-ABI declared in include/lbw_attn.h and include/lbw_gemm.h)."""
 import ctypes
 import os
 
@@ -37,6 +37,13 @@ SIGNATURES = {
                                  _p, _i64, _i64, _i64, _f32, _p, _p, _p]),
 }
 
+# the FP8 GEMM's entry points; mirrors include/lbw_gemm.h
+GEMM_SIGNATURES = {
+    "lbw_gemm_fp8_rows": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
+    "lbw_gemm_fp8_mx": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
+    "lbw_quant_mx_fp8_t": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _p]),
+}
+
 
 def sources_sha16():
     """First 16 hex digits of a sha256 over what liblbw_attn.so is built from: the HIP sources and headers (csrc/,
@@ -47,7 +54,7 @@ def sources_sha16():
     here = os.path.dirname(os.path.abspath(__file__))
     files = [os.path.join(here, "csrc", f) for f in sorted(os.listdir(os.path.join(here, "csrc")))
              if f.endswith((".hip", ".h"))]
-    files.append(os.path.join(os.path.dirname(here), "include", "lbw_attn.h"))
+    files += [os.path.join(os.path.dirname(here), "include", f) for f in ("lbw_attn.h", "lbw_gemm.h")]
     h = hashlib.sha256(" ".join(build.HIPCC_FLAGS).encode())
     for f in files:
         with open(f, "rb") as fh:
@@ -71,7 +78,7 @@ def load(path=LIB_PATH):
         raise ImportError(f"{path} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'` "
                           "or `python lingbot_world_v2_realtime_amd/build.py`")
     lib = ctypes.CDLL(path)
-    for name, (res, args) in SIGNATURES.items():
+    for name, (res, args) in (*SIGNATURES.items(), *GEMM_SIGNATURES.items()):
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args

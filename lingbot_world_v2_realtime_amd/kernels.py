@@ -329,10 +329,11 @@ def quant_rows_fp8_gelu(x):
     return x8, scale
 
 
-def quant_mx_fp8(x, rows_pad=None):
+def quant_mx_fp8(x, rows_pad=None, transposed=False):
     """MXFP8 of a 2-d bf16 / fp32 device tensor x [rows, cols] (cols a multiple of 32, unit column stride):
     (x8 float8_e4m3fn [rows_pad, cols], scale float8_e8m0fnu [rows_pad, cols / 32]), one power-of-two scale per 32
-    values; rows past `rows` (up to rows_pad, default rows) are zero with scale 1."""
+    values; rows past `rows` (up to rows_pad, default rows) are zero with scale 1. transposed (cols a multiple of
+    128): the scale bytes as uint8 [cols / 128, rows_pad, 4], the order gemm_fp8_mx takes."""
     lib = _lib.load()
     if not x.is_cuda:
         raise ValueError("x must be a device tensor (the FP8 path has no CPU implementation)")
@@ -343,11 +344,63 @@ def quant_mx_fp8(x, rows_pad=None):
     rows, cols = x.shape
     rows_pad = rows if rows_pad is None else int(rows_pad)
     x8 = torch.empty(rows_pad, cols, dtype=torch.float8_e4m3fn, device=x.device)
+    if transposed:
+        e8 = torch.empty(cols // 128, rows_pad, 4, dtype=torch.uint8, device=x.device)
+        st = lib.lbw_quant_mx_fp8_t(_ptr(x), int(x.dtype == torch.float32), rows, rows_pad, cols, x.stride(0),
+                                    _ptr(x8), _ptr(e8), _stream(x))
+        _lib.check(st, "lbw_quant_mx_fp8_t")
+        return x8, e8
     e8 = torch.empty(rows_pad, cols // 32, dtype=torch.uint8, device=x.device)
     st = lib.lbw_quant_mx_fp8(_ptr(x), int(x.dtype == torch.float32), rows, rows_pad, cols, x.stride(0), _ptr(x8),
                               _ptr(e8), _stream(x))
     _lib.check(st, "lbw_quant_mx_fp8")
     return x8, e8.view(torch.float8_e8m0fnu)
+
+
+def _gemm_operands(x8, w8, bias):
+    if x8.dtype != torch.float8_e4m3fn or w8.dtype != torch.float8_e4m3fn:
+        raise TypeError(f"x8 and w8 must be float8_e4m3fn, got {x8.dtype} / {w8.dtype}")
+    if x8.dim() != 2 or w8.dim() != 2 or x8.shape[1] != w8.shape[1] or not x8.is_contiguous() \
+            or not w8.is_contiguous():
+        raise ValueError(f"x8 {tuple(x8.shape)} and w8 {tuple(w8.shape)} must be contiguous [M, K] and [N, K]")
+    if bias is not None:
+        if bias.dtype != torch.bfloat16 or tuple(bias.shape) != (w8.shape[0],):
+            raise ValueError(f"bias must be bfloat16 ({w8.shape[0]},), got {bias.dtype} {tuple(bias.shape)}")
+        if not bias.is_contiguous() or bias.data_ptr() % 4:   # the kernel loads pairs
+            bias = bias.clone(memory_format=torch.contiguous_format)
+    return bias
+
+
+def gemm_fp8_rows(x8, x_scale, w8, w_scale, bias=None):
+    """The rowwise-scaled FP8 product (lbw_gemm_fp8_rows): x8 [M, K] and w8 [N, K] float8_e4m3fn, x_scale M and w_scale
+    N fp32 values, bias bf16 [N] or None -> bf16 [M, N] = x8 w8^T x_scale w_scale + bias, rounded once."""
+    m, n = x8.shape[0], w8.shape[0]
+    bias = _gemm_operands(x8, w8, bias)
+    if x_scale.dtype != torch.float32 or w_scale.dtype != torch.float32 or x_scale.numel() != m \
+            or w_scale.numel() != n or not x_scale.is_contiguous() or not w_scale.is_contiguous():
+        raise ValueError(f"scales must be {m} and {n} contiguous fp32 values")
+    _same_device("gemm_fp8_rows", x8, x_scale, w8, w_scale, bias)
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=x8.device)
+    st = _lib.load().lbw_gemm_fp8_rows(_ptr(x8), _ptr(x_scale), _ptr(w8), _ptr(w_scale), _ptr(bias), m, n,
+                                       x8.shape[1], _ptr(out), _stream(x8))
+    _lib.check(st, "lbw_gemm_fp8_rows")
+    return out
+
+
+def gemm_fp8_mx(x8, x_scale_t, w8, w_scale_t, bias=None):
+    """The MX-scaled FP8 product (lbw_gemm_fp8_mx): x8 [M, K] and w8 [N, K] float8_e4m3fn, their E8M0 scale bytes uint8
+    [K / 128, M, 4] and [K / 128, N, 4] (quant_mx_fp8(transposed=True)), bias bf16 [N] or None -> bf16 [M, N]."""
+    m, n, k = x8.shape[0], w8.shape[0], x8.shape[1]
+    bias = _gemm_operands(x8, w8, bias)
+    for s, rows in ((x_scale_t, m), (w_scale_t, n)):
+        if s.dtype != torch.uint8 or tuple(s.shape) != (k // 128, rows, 4) or not s.is_contiguous():
+            raise ValueError(f"scales must be contiguous uint8 {(k // 128, rows, 4)}, got {s.dtype} {tuple(s.shape)}")
+    _same_device("gemm_fp8_mx", x8, x_scale_t, w8, w_scale_t, bias)
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=x8.device)
+    st = _lib.load().lbw_gemm_fp8_mx(_ptr(x8), _ptr(x_scale_t), _ptr(w8), _ptr(w_scale_t), _ptr(bias), m, n, k,
+                                     _ptr(out), _stream(x8))
+    _lib.check(st, "lbw_gemm_fp8_mx")
+    return out
 
 
 _ATTN_WS = {}

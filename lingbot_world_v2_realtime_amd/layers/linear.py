@@ -3,10 +3,11 @@ output row, converted once at load; activations quantised per token on every cal
 scale per 32 values along K for both; the GEMM accumulates in fp32 and writes bf16.
 
 On MI355X the per-row quantisation of weights and activations is a HIP kernel (lbw_quant_rows_fp8, bit for bit the
-reference's formula) and the GEMM is hipBLASLt's rowwise-scaled FP8 GEMM, reached through torch._scaled_mm with the
-bias in its epilogue -- a plain library GEMM, which the dense FP8 MFMA path of the library already serves well.
-For the shapes in fp8_gemm_solutions.csv, use_tuned_gemms() makes the GEMM take the hipBLASLt solution measured
-fastest for that shape instead of the library's default pick (tune_gemms() writes such a table).
+reference's formula) and the GEMM another (lbw_gemm_fp8_rows / lbw_gemm_fp8_mx), with the scales and the bias in its
+epilogue. Only a rowwise call that records a gradient for the bias still runs hipBLASLt's
+rowwise-scaled FP8 GEMM through torch._scaled_mm, which autograd knows (and refuses to differentiate); for that call,
+and for a program's own _scaled_mm calls, use_tuned_gemms() picks the hipBLASLt solutions of fp8_gemm_solutions.csv
+(tune_gemms() writes such a table).
 """
 import os
 
@@ -85,14 +86,21 @@ class FP8Linear(torch.nn.Module):
             if x2.dtype not in (torch.bfloat16, torch.float32):
                 x2 = x2.float()
             x8, x_scale = kernels.quant_rows_fp8(x2.contiguous())
-        y = torch._scaled_mm(x8, self.w8.t(), scale_a=x_scale, scale_b=self.w_scale_t,
-                             bias=None if self.bias is None else self.bias.to(torch.bfloat16),
-                             out_dtype=torch.bfloat16)
+        bias = None if self.bias is None else self.bias.to(torch.bfloat16)
+        if _records_grad(bias) or not self.w8.is_contiguous() or self.out_features % 16:
+            y = torch._scaled_mm(x8, self.w8.t(), scale_a=x_scale, scale_b=self.w_scale_t, bias=bias,
+                                 out_dtype=torch.bfloat16)
+        else:
+            y = kernels.gemm_fp8_rows(x8, x_scale, self.w8, self.w_scale_t, bias)
         return y.reshape(*shape[:-1], y.shape[-1])
 
 
-MX_ROWS = 128   # hipBLASLt's MX-scaled GEMM takes row counts in multiples of its 128-row tile
-MX_K = 128      # and K in whole 128-value tiles: four E8M0 scale columns (the reference pads its scales to this too)
+def _records_grad(bias):
+    return bias is not None and bias.requires_grad and torch.is_grad_enabled()
+
+
+MX_ROWS = 128   # weight rows are padded to this (the library MX GEMM's row tile, which the stored weights keep)
+MX_K = 128      # K in whole 128-value tiles: four E8M0 scale columns (the reference pads its scales to this too)
 
 
 def _pad(n, m):
@@ -102,8 +110,8 @@ def _pad(n, m):
 class MXFP8Linear(torch.nn.Module):
     """MXFP8 replacement of an nn.Linear (lingbot/layers/linear.py:53-73): e4m3 with one power-of-two (E8M0)
     scale per 32 values along K for the weights (once) and the activations (every call). The quantisation is
-    lbw_quant_mx_fp8; the GEMM is hipBLASLt's MX-scaled FP8 GEMM, whose row counts are padded to 128 (the
-    quantiser writes the padding rows, so nothing is copied), the bias added after it as the reference does.
+    lbw_quant_mx_fp8 (the activations' scales in the GEMM's order: lbw_quant_mx_fp8_t), the GEMM lbw_gemm_fp8_mx with
+    the bias in its epilogue; a bias that records a gradient is added after it instead.
     A K that is not a multiple of 128 (the GEMM's scale tile) is padded with zero columns, weights once and
     activations per call: a zero group quantises to zeros, so the product is unchanged."""
 
@@ -119,8 +127,19 @@ class MXFP8Linear(torch.nn.Module):
         w8, ws = kernels.quant_mx_fp8(w.contiguous(), _pad(n, MX_ROWS))
         self.register_buffer("w8", w8)             # [Np, Kp]
         self.register_buffer("w_scale", ws)        # [Np, Kp / 32] e8m0
+        self.register_buffer("w_scale_t", None, persistent=False)   # the same bytes as the GEMM reads them
+        self._order_scales()
         self.bias = lin.bias
         self.in_features, self.out_features = lin.in_features, lin.out_features
+
+    def _order_scales(self):
+        """w_scale's bytes as [Kp / 128, Np, 4], made again whenever weights are loaded."""
+        n = self.w_scale.shape[0]
+        self.w_scale_t = self.w_scale.view(torch.uint8).view(n, -1, 4).transpose(0, 1).contiguous()
+
+    def _load_from_state_dict(self, *args, **kwargs):
+        super()._load_from_state_dict(*args, **kwargs)
+        self._order_scales()
 
     def forward(self, x):
         shape = x.shape
@@ -129,12 +148,13 @@ class MXFP8Linear(torch.nn.Module):
             x2 = x2.float()
         if self.k_pad:
             x2 = torch.nn.functional.pad(x2, (0, self.k_pad))
-        m = x2.shape[0]
-        x8, xs = kernels.quant_mx_fp8(x2.contiguous(), _pad(m, MX_ROWS))
-        y = torch._scaled_mm(x8, self.w8.t(), scale_a=xs, scale_b=self.w_scale, out_dtype=torch.bfloat16)
-        y = y[:m, :self.out_features]
-        if self.bias is not None:
-            y = y + self.bias.to(torch.bfloat16)
+        x8, xs = kernels.quant_mx_fp8(x2.contiguous(), transposed=True)
+        bias = None if self.bias is None else self.bias.to(torch.bfloat16)
+        fused = bias is not None and not _records_grad(bias) and self.out_features == self.w8.shape[0]
+        y = kernels.gemm_fp8_mx(x8, xs, self.w8, self.w_scale_t, bias if fused else None)
+        y = y[:, :self.out_features]
+        if bias is not None and not fused:
+            y = y + bias
         return y.reshape(*shape[:-1], self.out_features)
 
 
