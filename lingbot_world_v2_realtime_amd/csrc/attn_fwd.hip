@@ -41,22 +41,17 @@ struct AttnArgs {
   int seg_span[LBW_MAX_SEGMENTS];       // keys from the start of block seg_fb to the last attended key
   int seg_blk0[LBW_MAX_SEGMENTS + 1];   // first tile-relative block of each chunk; [n_seg] = nb
   int split0[XCDS_MAX + 1];             // split tiles of XCDs before x (prefix), for the merge grid
+  // XCD x's tiles are [t_lo[x], t_lo[x + 1]); those from ts[x] on are split, their units (tile, key block) dealt as
+  // contiguous ranges: units / gx = uq remainder ur
+  int t_lo[XCDS_MAX + 1], ts[XCDS_MAX], uq[XCDS_MAX], ur[XCDS_MAX];
+  float inv_gx;
 };
 
-// Range of tiles of XCD x and its data-parallel / split phases.
-struct XcdPlan {
-  int t_lo, t_hi, ts;   // tiles [t_lo, t_hi); tiles from ts on are split into pieces
-  int64_t units;        // (t_hi - ts) * nb
-};
-
-__device__ __forceinline__ XcdPlan xcd_plan(const AttnArgs& a, int x) {
-  XcdPlan p;
-  p.t_lo = (int)((int64_t)x * a.n_tiles / XCDS);
-  p.t_hi = (int)((int64_t)(x + 1) * a.n_tiles / XCDS);
-  const int rounds = (p.t_hi - p.t_lo) / a.gx;
-  p.ts = p.t_lo + rounds * a.gx;
-  p.units = (int64_t)(p.t_hi - p.ts) * a.nb;
-  return p;
+// First unit of workgroup i of XCD x in that XCD's split units: floor(i * units / gx), from the quotient and remainder
+// of units / gx (formed on the host: a 64-bit division is ~130 dependent instructions, and there were seven at the
+// start of every workgroup). i * ur < gx^2, so the float product's floor is exact.
+__device__ __forceinline__ int unit_lo(const AttnArgs& a, int x, int i) {
+  return i * a.uq[x] + (int)(((float)(i * a.ur[x]) + 0.5f) * a.inv_gx);
 }
 
 constexpr int S_MASKED = (int)0xFF800000;      // bits of -inf: the int max ignores it, exp2 gives 0
@@ -658,20 +653,20 @@ __device__ __forceinline__ void store_out(const AttnArgs& a, const Piece& st, ui
     }
 }
 
-// Part of a tile: o (unnormalised) and (m, l) per row into workspace slot (g, slot).
+// Part of a tile: o (unnormalised) and (m, l) per row into workspace slot (g, slot). The partials are laid out as the
+// registers hold them, [slot][wave][quad 4 mt + i][lane] float4, so every store (and the merge's every load) is 1 KB
+// contiguous; by rows, each store was 64 separate 16-byte pieces.
 __device__ __forceinline__ void store_part(const Piece& st, float* __restrict__ o_part, float* __restrict__ ml_part,
                                            int64_t slot_idx, int w) {
   const int lane = threadIdx.x & 63, lq = lane & 31, g = lane >> 5;
   const int row = w * 32 + lq;
-  float* op = o_part + (slot_idx * QT + row) * D;
+  float4* op = (float4*)o_part + ((slot_idx * AT_WAVES + w) * 16) * 64 + lane;
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ch = 32 * mt + 8 * i + 4 * g;
-      *(float4*)(op + ch) = make_float4(st.o[mt][4 * i], st.o[mt][4 * i + 1], st.o[mt][4 * i + 2],
-                                        st.o[mt][4 * i + 3]);
-    }
+    for (int i = 0; i < 4; ++i)
+      op[(4 * mt + i) * 64] = make_float4(st.o[mt][4 * i], st.o[mt][4 * i + 1], st.o[mt][4 * i + 2],
+                                          st.o[mt][4 * i + 3]);
   if (g == 0) *(float2*)(ml_part + (slot_idx * QT + row) * 2) = make_float2(st.m, st.l);
 }
 
@@ -690,117 +685,112 @@ __global__ __launch_bounds__(AT_THREADS, 1) void attn_fwd_kernel(const int8_t* _
   __shared__ __attribute__((aligned(1024))) uint8_t lds[AT_LDS];
   const int gid = blockIdx.x, x = gid % XCDS, i = gid / XCDS;
   const int w = threadIdx.x >> 6;
-  const XcdPlan p = xcd_plan(a, x);
-  Piece st;
-  // whole tiles, dealt round-robin among this XCD's workgroups
-  for (int tile = p.t_lo + i; tile < p.ts; tile += a.gx) {
-    const int bh = tile / a.q_tiles;
-    const int64_t q0 = (int64_t)(tile % a.q_tiles) * QT + w * 32;
-    attend_range<TWO, LOGITS>(a, q8, q_scale, bias, k8, k_scale, v8, v8lo, v_scale, lds, bh, q0, 0, a.nb, st, logits);
-    store_out(a, st, out, bh, q0);
-  }
-  // this workgroup's piece of the split tiles
-  if (p.units == 0) return;
-  const int64_t u0 = (int64_t)i * p.units / a.gx, u1 = (int64_t)(i + 1) * p.units / a.gx;
-  const int first_tile = p.ts + (int)(u0 / a.nb);
-  for (int64_t u = u0; u < u1;) {
-    const int tile = p.ts + (int)(u / a.nb);
-    const int j0 = (int)(u % a.nb);
-    const int j1 = (int)((u1 - u + j0 < a.nb) ? (u1 - u + j0) : a.nb);
-    const int bh = tile / a.q_tiles;
-    const int64_t q0 = (int64_t)(tile % a.q_tiles) * QT + w * 32;
-    attend_range<TWO, LOGITS>(a, q8, q_scale, bias, k8, k_scale, v8, v8lo, v_scale, lds, bh, q0, j0, j1, st, logits);
-    if (j0 == 0 && j1 == a.nb) {
-      store_out(a, st, out, bh, q0);
-    } else {
-      store_part(st, o_part, ml_part, (int64_t)gid * 2 + (tile == first_tile ? 0 : 1), w);
+  // whole tiles, dealt round-robin among this XCD's workgroups, then this workgroup's piece of the split tiles: one
+  // loop, so the block loop's code is there once (two copies were 29 KB of a 64 KB instruction cache)
+  const int ts = a.ts[x];
+  int tile = a.t_lo[x] + i, j0 = 0, left = 0, first_tile = -1;
+  for (;;) {
+    int j1 = a.nb;
+    if (tile >= ts) {
+      if (first_tile < 0) {
+        const int u0 = unit_lo(a, x, i);
+        left = unit_lo(a, x, i + 1) - u0;
+        const int tt = (int)((uint32_t)u0 / (uint32_t)a.nb);
+        first_tile = tile = ts + tt;
+        j0 = u0 - tt * a.nb;
+      }
+      if (left <= 0) return;
+      j1 = left + j0 < a.nb ? left + j0 : a.nb;
+      left -= j1 - j0;
     }
-    u += j1 - j0;
+    const int bh = (int)((uint32_t)tile / (uint32_t)a.q_tiles);
+    const int64_t q0 = (int64_t)(tile - bh * a.q_tiles) * QT + w * 32;
+    Piece st;
+    attend_range<TWO, LOGITS>(a, q8, q_scale, bias, k8, k_scale, v8, v8lo, v_scale, lds, bh, q0, j0, j1, st, logits);
+    if (j0 == 0 && j1 == a.nb) store_out(a, st, out, bh, q0);
+    else store_part(st, o_part, ml_part, (int64_t)gid * 2 + (tile == first_tile ? 0 : 1), w);
+    if (first_tile < 0) tile += a.gx;
+    else ++tile;
+    j0 = 0;
   }
 }
 
 // Combine the pieces of each split tile: O = sum 2^(m_i - M) o_i / sum 2^(m_i - M) l_i
-// (experiments/bench_attn/splitkv/README.md:62). Grid: (split tile, 16-row slab) -- only split tiles are
-// launched; 256 threads = 16 rows x 16 lanes, each lane 8 consecutive channels, so a row's 512-byte partial is
-// read by 16 consecutive lanes.
-constexpr int MERGE_ROWS = 16;
+// (experiments/bench_attn/splitkv/README.md:62). Grid: (split tile, wave of the tile, mt) -- only split tiles are
+// launched; wave i of the 256 threads merges quad 4 mt + i, one float4 a lane, in the partials' register layout. The
+// pieces are read four at a time and merged online (running max), so their loads and (m, l) arrive together. Bound by
+// the latency of its few dependent loads: 8 tiles in 32 pieces each (33 MB) 17.0 -> 8.2 us, in 8 pieces 11.0 -> 9.7 us,
+// against 16-row slabs of the row layout that read every (m, l) in a pass of its own.
+constexpr int MERGE_WGS = AT_WAVES * 4;
+constexpr int MERGE_N = 4;
 __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict__ o_part,
                                                          const float* __restrict__ ml_part,
                                                          uint16_t* __restrict__ out, AttnArgs a) {
-  const int st = blockIdx.x / (QT / MERGE_ROWS), slab = blockIdx.x % (QT / MERGE_ROWS);
+  const int st = blockIdx.x / MERGE_WGS, w = blockIdx.x / 4 % AT_WAVES, mt = blockIdx.x & 3;
   int x = 0;
   while (x + 1 < XCDS && st >= a.split0[x + 1]) ++x;
-  const XcdPlan p = xcd_plan(a, x);
-  const int tile = p.ts + (st - a.split0[x]);
-  const int64_t ua = (int64_t)(tile - p.ts) * a.nb, ub = ua + a.nb;
-  // workgroups of this XCD whose unit range meets [ua, ub): owner(u) = floor(((u + 1) gx - 1) / units)
-  const int i_a = (int)(((ua + 1) * a.gx - 1) / p.units);
-  const int i_b = (int)((ub * a.gx - 1) / p.units);
-  // workgroup i's units are [floor(i units / gx), floor((i + 1) units / gx)): stepped from i_a with the quotient
-  // and remainder of units / gx, so the loops below divide nothing (64-bit divisions are long instruction
-  // sequences, and this kernel is short)
-  const int64_t uq = p.units / a.gx;
-  const int ur = (int)(p.units % a.gx);
-  const int64_t lo_a = (int64_t)i_a * uq + (int64_t)i_a * ur / a.gx;
-  const int rem_a = (int)((int64_t)i_a * ur % a.gx);
-  const int64_t hi_a = lo_a + uq + (rem_a + ur >= a.gx ? 1 : 0);
-  if (i_a == i_b && lo_a <= ua && hi_a >= ub) return;   // written whole by one workgroup
-  const int t = threadIdx.x, row = slab * MERGE_ROWS + (t >> 4), c0 = (t & 15) * 8;
-  const int64_t q = (int64_t)(tile % a.q_tiles) * QT + row;
+  const int rel = st - a.split0[x], tile = a.ts[x] + rel, ua = rel * a.nb, ub = ua + a.nb;
+  // workgroup of unit u: the last one whose first unit is at most u (estimated in float, then stepped to it)
+  const auto owner = [&](int u) {
+    int k = (int)((float)u / ((float)a.uq[x] + (float)a.ur[x] * a.inv_gx));
+    k = k < a.gx ? k : a.gx - 1;
+    while (unit_lo(a, x, k) > u) --k;
+    while (k + 1 < a.gx && unit_lo(a, x, k + 1) <= u) ++k;
+    return k;
+  };
+  const int i_a = owner(ua), i_b = owner(ub - 1);
+  if (i_a == i_b && unit_lo(a, x, i_a) <= ua) return;   // written whole by one workgroup
+  const int lane = threadIdx.x & 63, lq = lane & 31, g = lane >> 5, i = threadIdx.x >> 6;
+  const int row = w * 32 + lq;
+  const int bh = (int)((uint32_t)tile / (uint32_t)a.q_tiles);
+  const int64_t q = (int64_t)(tile - bh * a.q_tiles) * QT + row;
+  // a piece of workgroup ii that meets this tile is in its partial slot 0 when the tile is the first of the
+  // workgroup's range, i.e. when its range starts inside the tile, else in slot 1. Loads of a workgroup past i_b are
+  // replaced by i_b's, and a workgroup without units here counts as m = -inf (select, not multiply: its slot may hold
+  // anything).
+  const float4* op = (const float4*)o_part + (w * 16 + 4 * mt + i) * 64 + lane;
+  float m = -INFINITY, den = 0.f;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int i0 = i_a; i0 <= i_b; i0 += MERGE_N) {
+    float2 ml[MERGE_N];
+    float4 v[MERGE_N];
+    float mb = m;
+#pragma unroll
+    for (int n = 0; n < MERGE_N; ++n) {
+      const int ii = i0 + n <= i_b ? i0 + n : i_b;
+      const int64_t slot = (int64_t)(ii * XCDS + x) * 2 + (unit_lo(a, x, ii) >= ua ? 0 : 1);
+      ml[n] = *(const float2*)(ml_part + (slot * QT + row) * 2);
+      v[n] = op[slot * (AT_WAVES * 16 * 64)];
+    }
+#pragma unroll
+    for (int n = 0; n < MERGE_N; ++n) {
+      const int ii = i0 + n <= i_b ? i0 + n : i_b;
+      const int lo = unit_lo(a, x, ii), hi = unit_lo(a, x, ii + 1);
+      if (i0 + n > i_b || hi <= lo) ml[n] = make_float2(-INFINITY, 0.f), v[n] = make_float4(0.f, 0.f, 0.f, 0.f);
+      mb = fmaxf(mb, ml[n].x);
+    }
+    // the first batch holds workgroup i_a's piece, so mb is its rows' finite max from here on
+    const float keep = __builtin_amdgcn_exp2f(m - mb);
+    den *= keep;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] *= keep;
+#pragma unroll
+    for (int n = 0; n < MERGE_N; ++n) {
+      const float wgt = __builtin_amdgcn_exp2f(ml[n].x - mb);
+      den += wgt * ml[n].y;
+      acc[0] += wgt * v[n].x; acc[1] += wgt * v[n].y; acc[2] += wgt * v[n].z; acc[3] += wgt * v[n].w;
+    }
+    m = mb;
+  }
   if (q >= a.lq) return;
-  // a piece of workgroup ii that meets this tile is in its partial slot 0 when the tile is the first of
-  // the workgroup's range, i.e. when the piece starts inside the tile, else in slot 1
-  // The loads do not depend on whether workgroup ii's range meets the tile (every slot index stays inside the
-  // workspace, ii < gx), so they are issued unconditionally and unrolled to keep several in flight; a slot of a
-  // workgroup with no units here is read but not used (select, not multiply: it may hold anything).
-  float mmax = -INFINITY;
-  {
-    int64_t lo = lo_a;
-    int rem = rem_a;
-#pragma unroll 8
-    for (int ii = i_a; ii <= i_b; ++ii) {
-      const bool carry = rem + ur >= a.gx;
-      const int64_t hi = lo + uq + (carry ? 1 : 0);
-      rem += ur - (carry ? a.gx : 0);
-      const int64_t slot = (int64_t)(ii * XCDS + x) * 2 + (lo >= ua ? 0 : 1);
-      const float m = ml_part[(slot * QT + row) * 2];
-      if (hi > lo && hi > ua && lo < ub) mmax = fmaxf(mmax, m);   // units of this tile
-      lo = hi;
-    }
-  }
-  float acc[8], den = 0.f;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] = 0.f;
-  int64_t lo = lo_a;
-  int rem = rem_a;
-#pragma unroll 8
-  for (int ii = i_a; ii <= i_b; ++ii) {
-    const bool carry = rem + ur >= a.gx;
-    const int64_t hi = lo + uq + (carry ? 1 : 0);
-    rem += ur - (carry ? a.gx : 0);
-    const int64_t plo = lo;
-    lo = hi;
-    const int64_t slot = (int64_t)(ii * XCDS + x) * 2 + (plo >= ua ? 0 : 1);
-    const float2 ml = *(const float2*)(ml_part + (slot * QT + row) * 2);
-    const float* op = o_part + (slot * QT + row) * D + c0;
-    const float4 v0 = *(const float4*)op, v1 = *(const float4*)(op + 4);
-    if (hi > plo && hi > ua && plo < ub) {
-      const float wgt = __builtin_amdgcn_exp2f(ml.x - mmax);
-      den += wgt * ml.y;
-      acc[0] += wgt * v0.x; acc[1] += wgt * v0.y; acc[2] += wgt * v0.z; acc[3] += wgt * v0.w;
-      acc[4] += wgt * v1.x; acc[5] += wgt * v1.y; acc[6] += wgt * v1.z; acc[7] += wgt * v1.w;
-    }
-  }
   const float inv = 1.f / den;
-  const int bh = tile / a.q_tiles;
-  const int64_t b = bh / a.heads, h = bh % a.heads;
-  uint16_t* dst = out + b * a.o_sb + q * a.o_st + h * a.o_sh + c0;
-  uint32_t w[4];
+  const int64_t b = bh / a.heads, h = bh - b * a.heads;
+  uint16_t* dst = out + b * a.o_sb + q * a.o_st + h * a.o_sh + 32 * mt + 8 * i + 4 * g;
+  uint32_t o2[2];
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
-    w[c] = f32_to_bf16_bits(acc[2 * c] * inv) | ((uint32_t)f32_to_bf16_bits(acc[2 * c + 1] * inv) << 16);
-  *(uint2*)dst = make_uint2(w[0], w[1]);        // the output contract guarantees 8-byte alignment
-  *(uint2*)(dst + 4) = make_uint2(w[2], w[3]);
+  for (int c = 0; c < 2; ++c)
+    o2[c] = f32_to_bf16_bits(acc[2 * c] * inv) | ((uint32_t)f32_to_bf16_bits(acc[2 * c + 1] * inv) << 16);
+  *(uint2*)dst = make_uint2(o2[0], o2[1]);   // the output contract guarantees 8-byte alignment
 }
 
 // Persistent workgroups per XCD: one per CU (a workgroup is 8 waves, two per SIMD, and uses AT_LDS bytes of the
@@ -879,10 +869,16 @@ static int attn_launch(const int8_t* q8, const float* q_scale, const float* bias
   a.n_tiles = (int)(a.q_tiles * a.bh);
   if (const int dv = check_device()) return dv;
   a.gx = attn_wgs_per_xcd();
+  a.inv_gx = 1.f / (float)a.gx;
   a.split0[0] = 0;
-  for (int x = 0; x < XCDS; ++x) {   // tiles past the whole-tile rounds of each XCD are split (xcd_plan)
-    const int t_lo = (int)((int64_t)x * a.n_tiles / XCDS), t_hi = (int)((int64_t)(x + 1) * a.n_tiles / XCDS);
-    a.split0[x + 1] = a.split0[x] + (t_hi - t_lo) % a.gx;
+  if ((int64_t)a.gx * a.nb > 0x7fffffff) return LBW_E_SHAPE;   // split units of an XCD in 31 bits
+  for (int x = 0; x <= XCDS; ++x) a.t_lo[x] = (int)((int64_t)x * a.n_tiles / XCDS);
+  for (int x = 0; x < XCDS; ++x) {   // tiles past the whole-tile rounds of each XCD are split
+    const int split = (a.t_lo[x + 1] - a.t_lo[x]) % a.gx;
+    a.ts[x] = a.t_lo[x + 1] - split;
+    a.uq[x] = (int)((int64_t)split * a.nb / a.gx);
+    a.ur[x] = (int)((int64_t)split * a.nb % a.gx);
+    a.split0[x + 1] = a.split0[x] + split;
   }
   float* o_part = (float*)workspace;
   float* ml_part = o_part + (int64_t)XCDS * a.gx * 2 * QT * D;
@@ -901,7 +897,7 @@ static int attn_launch(const int8_t* q8, const float* q_scale, const float* bias
     hipLaunchKernelGGL((attn_fwd_kernel<false, false>), grid, block, 0, st, q8, q_scale, bias, k8, k_scale, v8, v8lo,
                        v_scale, out, o_part, ml_part, logits, a);
   if (a.split0[XCDS] > 0)
-    hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)(a.split0[XCDS] * (QT / MERGE_ROWS))), dim3(256), 0, st,
+    hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)(a.split0[XCDS] * MERGE_WGS)), dim3(256), 0, st,
                        o_part, ml_part, out, a);
   if (hipGetLastError() != hipSuccess) return LBW_E_LAUNCH;
   return LBW_OK;
