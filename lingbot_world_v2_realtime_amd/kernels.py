@@ -20,12 +20,24 @@ def pad_to(n, m):
     return (n + m - 1) // m * m
 
 
+# The short calls are bound by this module's own Python, so it keeps to what a call needs: the current stream's handle
+# without a Stream object (0.2 against 1.6 us), layers of the ring as pointer offsets instead of indexed views (~1.5 us
+# each, eleven in a write and an attention), device numbers instead of sets of device objects.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # (torch builds without a GPU backend have none)
+_I32_ARRAYS = [ctypes_i32 * n for n in range(MAX_SEGMENTS + 1)]
+
+
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def _ptr(t):
     return t.data_ptr() if t is not None else None
+
+
+def _i32_array(vals):
+    n = len(vals)
+    return (_I32_ARRAYS[n] if n <= MAX_SEGMENTS else ctypes_i32 * n)(*vals)
 
 
 def _require_cuda_bf16(name, t):
@@ -43,15 +55,28 @@ DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1}   # LBW_DTYPE_BF16 / LBW_DTYP
 def _require_cuda_16(name, t):
     """A device tensor of bf16 or fp16 with a contiguous 128-wide head dim (the quantisers' inputs); returns the
     format code the C-ABI takes."""
-    if t.dtype not in DTYPE_CODE:
+    code = DTYPE_CODE.get(t.dtype)
+    if code is None:
         raise TypeError(f"{name} must be bfloat16 or float16, got {t.dtype}")
-    _require_cuda_bf16(name, t.view(torch.bfloat16) if t.dtype == torch.float16 else t)
-    return DTYPE_CODE[t.dtype]
+    if not t.is_cuda or t.shape[-1] != HEAD_DIM or t.stride(-1) != 1:
+        _require_cuda_bf16(name, t.view(torch.bfloat16) if code else t)
+    return code
 
 
 def _same_device(what, *tensors):
     """Every tensor (None skipped) on one device: a kernel launched on the current device would otherwise read or
     write another GPU's memory through a raw pointer."""
+    first = None
+    for t in tensors:
+        if t is None:
+            continue
+        d = t.get_device()   # -1 off the GPU, whichever device that is
+        if first is None:
+            first = d
+        if d != first or d < 0:
+            break
+    else:
+        return
     devs = {t.device for t in tensors if t is not None}
     if len(devs) > 1:
         raise ValueError(f"{what}: tensors on different devices {sorted(str(d) for d in devs)}")
@@ -94,6 +119,17 @@ class RingCache:
     def bh(self):
         return self.batch * self.heads
 
+    def layer_ptrs(self, layer):
+        """Device addresses of one layer's (k8, k_scale, km, v8, v8lo or None, v_scale)."""
+        if not -self.layers <= layer < self.layers:
+            raise IndexError(f"layer {layer} is out of range for {self.layers} layers")
+        i = layer + self.layers if layer < 0 else layer
+        lo = self.v8lo
+        return (self.k8.data_ptr() + i * self.k8.stride(0), self.k_scale.data_ptr() + 4 * i * self.k_scale.stride(0),
+                self.km.data_ptr() + 4 * i * self.km.stride(0), self.v8.data_ptr() + i * self.v8.stride(0),
+                lo.data_ptr() + i * lo.stride(0) if lo is not None else None,
+                self.v_scale.data_ptr() + i * self.v_scale.stride(0))
+
     def layer_view(self, layer):
         """(k8, k_scale, km, v8, v8lo or None, v_scale) of one layer, for the per-layer entry points."""
         return (self.k8[layer], self.k_scale[layer], self.km[layer], self.v8[layer],
@@ -118,20 +154,20 @@ def kv_requant(k, v, ring, slot, layer0=0, workspace=None):
     if k.shape != v.shape:
         raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} differ")
     _same_device("kv_requant", k, v, ring.k8, workspace)
+    ks, vs = k.stride(), v.stride()
     if k.dim() == 4:
-        k, v = k.unsqueeze(0), v.unsqueeze(0)
-    nl, b, n, h, _ = k.shape
+        nl, (b, n, h, _) = 1, k.shape
+        ks, vs = (0,) + ks, (0,) + vs
+    else:
+        nl, b, n, h, _ = k.shape
     if b != ring.batch or h != ring.heads or n > ring.cap or layer0 + nl > ring.layers:
         raise ValueError(f"chunk {tuple(k.shape)} does not fit the ring "
                          f"(layers {ring.layers}, batch {ring.batch}, heads {ring.heads}, cap {ring.cap})")
     if workspace is None:
         workspace = requant_workspace(nl, b * h, n, k.device)
-    ks, vs = k.stride(), v.stride()
     st = lib.lbw_kv_requant(
-        _ptr(k), _ptr(v), dtype, nl, b, n, h, ks[0], ks[1], ks[2], ks[3], vs[0], vs[1], vs[2], vs[3],
-        _ptr(ring.k8[layer0]), _ptr(ring.k_scale[layer0]), _ptr(ring.km[layer0]), _ptr(ring.v8[layer0]),
-        _ptr(ring.v8lo[layer0]) if ring.v8lo is not None else None, _ptr(ring.v_scale[layer0]),
-        ring.slots, ring.cap, slot, _ptr(workspace), _stream(k))
+        k.data_ptr(), v.data_ptr(), dtype, nl, b, n, h, ks[0], ks[1], ks[2], ks[3], vs[0], vs[1], vs[2], vs[3],
+        *ring.layer_ptrs(layer0), ring.slots, ring.cap, slot, workspace.data_ptr(), _stream(k))
     _lib.check(st, "lbw_kv_requant")
 
 
@@ -150,8 +186,8 @@ def quant_q(q, layout="NHD", ring=None, layer=0, seg_slots=()):
     km_ptr, slots, seg_arr = None, 1, None
     if n_seg > 1:
         bias = torch.empty(n_seg, bh, lp, dtype=torch.float32, device=q.device)
-        km_ptr, slots = _ptr(ring.km[layer]), ring.slots
-        seg_arr = (ctypes_i32 * n_seg)(*seg_slots)
+        km_ptr, slots = ring.layer_ptrs(layer)[2], ring.slots
+        seg_arr = _i32_array(seg_slots)
     st = lib.lbw_quant_q(_ptr(q), dtype, b, lq, h, s_b, s_t, s_h, _ptr(q8), _ptr(qs), km_ptr, slots, n_seg,
                          seg_arr, _ptr(bias), _stream(q))
     _lib.check(st, "lbw_quant_q")
@@ -196,8 +232,8 @@ def norm_rope_quant_q(q, heads, weight, eps, rope, ring=None, layer=0, seg_slots
     bias, km_ptr, slots, seg_arr = None, None, 1, None
     if n_seg > 1:
         bias = torch.empty(n_seg, bh, lp, dtype=torch.float32, device=q.device)
-        km_ptr, slots = _ptr(ring.km[layer]), ring.slots
-        seg_arr = (ctypes_i32 * n_seg)(*seg_slots)
+        km_ptr, slots = ring.layer_ptrs(layer)[2], ring.slots
+        seg_arr = _i32_array(seg_slots)
     roped = torch.empty(b, lq, heads, HEAD_DIM, dtype=torch.bfloat16, device=q.device) if want_roped else None
     os_ = roped.stride()[:3] if roped is not None else (0, 0, 0)
     st = lib.lbw_norm_rope_quant_q(_ptr(q), b, lq, heads, q.stride(0), q.stride(1), _ptr(weight), float(eps),
@@ -230,13 +266,11 @@ def norm_rope_kv_requant(k, v, heads, weight, eps, rope, ring, slot, layer=0, k_
         raise ValueError(f"k_out {tuple(k_out.shape)} must be {(b, n, heads, HEAD_DIM)}")
     if workspace is None:
         workspace = requant_workspace(1, b * heads, n, k.device)
-    k8, ksc, km, v8, v8lo, vsc = ring.layer_view(layer)
     vs, os_ = v.stride(), k_out.stride()
     st = lib.lbw_norm_rope_kv_requant(_ptr(k), _ptr(v), b, n, heads, k.stride(0), k.stride(1), vs[0], vs[1], vs[2],
                                       _ptr(weight), float(eps), _ptr(rope.table), rope.table.shape[0], rope.grid_h,
-                                      rope.grid_w, rope.start_frame, _ptr(k_out), os_[0], os_[1], os_[2], _ptr(k8),
-                                      _ptr(ksc), _ptr(km), _ptr(v8), _ptr(v8lo), _ptr(vsc), ring.slots, ring.cap,
-                                      slot, _ptr(workspace), _stream(k))
+                                      rope.grid_w, rope.start_frame, _ptr(k_out), os_[0], os_[1], os_[2],
+                                      *ring.layer_ptrs(layer), ring.slots, ring.cap, slot, _ptr(workspace), _stream(k))
     _lib.check(st, "lbw_norm_rope_kv_requant")
     return k_out
 
@@ -414,11 +448,15 @@ def attn_workspace(device, stream=None):
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
     if stream is None:
         stream = torch.cuda.current_stream(idx).cuda_stream
-    key = (dev.type, idx, stream)
-    if key not in _ATTN_WS:
+    return _attn_workspace(idx, stream)
+
+
+def _attn_workspace(idx, stream):
+    ws = _ATTN_WS.get((idx, stream))
+    if ws is None:
         nbytes = _lib.load().lbw_attn_workspace_bytes()
-        _ATTN_WS[key] = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=torch.device(dev.type, idx))
-    return _ATTN_WS[key]
+        ws = _ATTN_WS[idx, stream] = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=torch.device("cuda", idx))
+    return ws
 
 
 def key_blocks(seg_lens, seg_firsts=None):
@@ -441,9 +479,9 @@ def attn_fwd(q8, q_scale, bias, batch, lq, heads, ring, layer, seg_slots, seg_le
         raise ValueError(f"need 1..{MAX_SEGMENTS} chunks with a length each, got {seg_slots} / {seg_lens}")
     if seg_firsts is not None and len(seg_firsts) != n_seg:
         raise ValueError(f"need a first token per chunk, got {seg_firsts} for {n_seg} chunks")
-    if any(int(n) < 1 for n in seg_lens) or any(int(f) < 0 or int(f) + int(n) > ring.cap for f, n in
-                                                zip(seg_firsts or [0] * n_seg, seg_lens)):
-        raise ValueError(f"chunk ranges (first {seg_firsts}, length {seg_lens}) must lie in slots of {ring.cap}")
+    for f, n in zip(seg_firsts or [0] * n_seg, seg_lens):
+        if int(n) < 1 or int(f) < 0 or int(f) + int(n) > ring.cap:
+            raise ValueError(f"chunk ranges (first {seg_firsts}, length {seg_lens}) must lie in slots of {ring.cap}")
     _require_cuda_bf16("out", out)
     _same_device("attn_fwd", q8, q_scale, bias, out, ring.k8, workspace)
     ob, ol, oh, o_b, o_t, o_h = _dims(out, layout)
@@ -466,34 +504,34 @@ def attn_fwd(q8, q_scale, bias, batch, lq, heads, ring, layer, seg_slots, seg_le
         raise ValueError(f"{n_seg} chunks need a contiguous fp32 bias ({n_seg}, {bh}, {lp}), got "
                          f"{None if bias is None else tuple(bias.shape)}")
     sm_scale = HEAD_DIM ** -0.5 if sm_scale is None else float(sm_scale)
-    k8, ksc, _, v8, v8lo, vsc = ring.layer_view(layer)
-    slot_arr = (ctypes_i32 * n_seg)(*seg_slots)
-    len_arr = (ctypes_i32 * n_seg)(*seg_lens)
-    first_arr = (ctypes_i32 * n_seg)(*seg_firsts) if seg_firsts is not None else None
+    k8, ksc, _, v8, v8lo, vsc = ring.layer_ptrs(layer)
+    slot_arr, len_arr = _i32_array(seg_slots), _i32_array(seg_lens)
+    first_arr = _i32_array(seg_firsts) if seg_firsts is not None else None
+    stream = _stream(q8)
     if noalloc:
         if logits is not None:
             raise ValueError("the checking build runs through lbw_qk_logits_i32, which takes a workspace")
-        st = lib.lbw_attn_fwd_noalloc(_ptr(q8), _ptr(q_scale), _ptr(bias), batch, lq, heads, _ptr(k8), _ptr(ksc),
-                                      _ptr(v8), _ptr(v8lo), _ptr(vsc), ring.slots, ring.cap, n_seg, slot_arr, len_arr,
-                                      first_arr, _ptr(out), o_b, o_t, o_h, sm_scale, _stream(q8))
+        st = lib.lbw_attn_fwd_noalloc(_ptr(q8), _ptr(q_scale), _ptr(bias), batch, lq, heads, k8, ksc,
+                                      v8, v8lo, vsc, ring.slots, ring.cap, n_seg, slot_arr, len_arr,
+                                      first_arr, _ptr(out), o_b, o_t, o_h, sm_scale, stream)
         _lib.check(st, "lbw_attn_fwd_noalloc")
         return out
     if workspace is None:
-        workspace = attn_workspace(q8.device, _stream(q8))
+        workspace = _attn_workspace(q8.get_device(), stream)
     if logits is not None:
         want = (bh, lp, K_BLOCK * key_blocks(seg_lens, seg_firsts))
         if logits.dtype != torch.int32 or tuple(logits.shape) != want or not logits.is_contiguous():
             raise ValueError(f"logits must be contiguous int32 {want}, got {logits.dtype} {tuple(logits.shape)}")
         _same_device("qk_logits", q8, logits)
-        st = lib.lbw_qk_logits_i32(_ptr(q8), _ptr(q_scale), _ptr(bias), batch, lq, heads, _ptr(k8), _ptr(ksc),
-                                   _ptr(v8), _ptr(v8lo), _ptr(vsc), ring.slots, ring.cap, n_seg, slot_arr, len_arr,
+        st = lib.lbw_qk_logits_i32(_ptr(q8), _ptr(q_scale), _ptr(bias), batch, lq, heads, k8, ksc,
+                                   v8, v8lo, vsc, ring.slots, ring.cap, n_seg, slot_arr, len_arr,
                                    first_arr, _ptr(out), o_b, o_t, o_h, sm_scale, _ptr(logits), _ptr(workspace),
-                                   _stream(q8))
+                                   stream)
         _lib.check(st, "lbw_qk_logits_i32")
         return out
-    st = lib.lbw_attn_fwd(_ptr(q8), _ptr(q_scale), _ptr(bias), batch, lq, heads, _ptr(k8), _ptr(ksc),
-                          _ptr(v8), _ptr(v8lo), _ptr(vsc), ring.slots, ring.cap, n_seg, slot_arr, len_arr, first_arr,
-                          _ptr(out), o_b, o_t, o_h, sm_scale, _ptr(workspace), _stream(q8))
+    st = lib.lbw_attn_fwd(_ptr(q8), _ptr(q_scale), _ptr(bias), batch, lq, heads, k8, ksc,
+                          v8, v8lo, vsc, ring.slots, ring.cap, n_seg, slot_arr, len_arr, first_arr,
+                          _ptr(out), o_b, o_t, o_h, sm_scale, _ptr(workspace), stream)
     _lib.check(st, "lbw_attn_fwd")
     return out
 
@@ -519,10 +557,10 @@ def _dims(x, layout):
     """(B, L, H, stride_batch, stride_tok, stride_head) of an NHD [B, L, H, D] or HND [B, H, L, D] tensor."""
     if x.dim() != 4:
         raise ValueError(f"expected a 4-d tensor, got shape {tuple(x.shape)}")
-    s = x.stride()
+    (a, b, c, _), s = x.shape, x.stride()
     if layout == "NHD":
-        return x.shape[0], x.shape[1], x.shape[2], s[0], s[1], s[2]
+        return a, b, c, s[0], s[1], s[2]
     if layout == "HND":
-        return x.shape[0], x.shape[2], x.shape[1], s[0], s[2], s[1]
+        return a, c, b, s[0], s[2], s[1]
     raise ValueError(f"tensor_layout must be 'NHD' or 'HND', got {layout!r}")
 

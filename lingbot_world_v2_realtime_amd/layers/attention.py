@@ -27,9 +27,9 @@ _DROPIN = {}
 
 
 def _dropin_buffers(b, h, lk, device):
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    key = (b, h, idx, torch.cuda.current_stream(idx).cuda_stream)
+    key = (b, h, idx, kernels._raw_stream(idx))
     held = _DROPIN.get(key)
     if held is None or held[0].cap < lk:
         cap = kernels.pad_to(lk, kernels.K_BLOCK)
@@ -50,8 +50,9 @@ def sage_attention(q, k, v, tensor_layout="NHD", is_causal=False, sm_scale=None)
     """
     if is_causal:
         raise NotImplementedError("the quantized kernel is non-causal; the DiT never calls it causally")
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        kernels._require_cuda_16(name, t)
+    kernels._require_cuda_16("q", q)
+    kernels._require_cuda_16("k", k)
+    kernels._require_cuda_16("v", v)
     b, lq, h, *_ = kernels._dims(q, tensor_layout)
     bk, lk, hk, *_ = kernels._dims(k, tensor_layout)
     if (bk, hk) != (b, h) or tuple(v.shape) != tuple(k.shape):
@@ -91,20 +92,26 @@ def flash_attention(q, k, v, k_lens=None, **kw):
     q.dtype. Inputs that are not fp16 / bf16 are cast to `dtype` first, as the reference does; the kernel computes
     in bf16. Calls with arguments the kernel does not take (q_lens, dropout, causal, a window, q_scale) get the
     paper's SDPA form instead."""
-    opts = {key: kw.get(key, dflt) for key, dflt in _FLASH_DEFAULTS.items()}
-    dtype = kw.get("dtype", torch.bfloat16)
-    if any(opts[key] != dflt for key, dflt in _FLASH_DEFAULTS.items() if key != "window_size") or \
-            tuple(opts["window_size"]) != (-1, -1) or q.shape[-1] != kernels.HEAD_DIM:
+    dtype = torch.bfloat16
+    if kw:
+        opts = {key: kw.get(key, dflt) for key, dflt in _FLASH_DEFAULTS.items()}
+        dtype = kw.get("dtype", torch.bfloat16)
+        if any(opts[key] != dflt for key, dflt in _FLASH_DEFAULTS.items() if key != "window_size") or \
+                tuple(opts["window_size"]) != (-1, -1):
+            return _paper_attention(q, k, v, k_lens=k_lens, **kw)
+    if q.shape[-1] != kernels.HEAD_DIM:
         return _paper_attention(q, k, v, k_lens=k_lens, **kw)
     out_dtype = q.dtype
 
     def half(x):
-        return x if x.dtype in (torch.float16, torch.bfloat16) else x.to(dtype)
+        if x.dtype == torch.bfloat16:
+            return x
+        return (x if x.dtype == torch.float16 else x.to(dtype)).to(torch.bfloat16)
 
-    qh, kh, vh = (half(x).to(torch.bfloat16) for x in (q, k, v))
+    qh, kh, vh = half(q), half(k), half(v)
     ctx = kernels.CrossContext(kh, vh)
     out = kernels.cross_attn_fwd(qh, ctx, sm_scale=kw.get("softmax_scale"), k_lens=k_lens)
-    return out.to(out_dtype)
+    return out if out.dtype == out_dtype else out.to(out_dtype)
 
 
 class CrossAttnCache:

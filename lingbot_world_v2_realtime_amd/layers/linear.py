@@ -92,7 +92,7 @@ class FP8Linear(torch.nn.Module):
                                  out_dtype=torch.bfloat16)
         else:
             y = kernels.gemm_fp8_rows(x8, x_scale, self.w8, self.w_scale_t, bias)
-        return y.reshape(*shape[:-1], y.shape[-1])
+        return y if len(shape) == 2 else y.view(*shape[:-1], y.shape[1])
 
 
 def _records_grad(bias):
