@@ -1,6 +1,6 @@
 // K/V re-quant of finished chunks into the quantised ring cache (gfx950).
 //
-// Three launches:
+// Three launches (two for short chunks):
 //   1. kv_stats:    per 64-token block (grid: block, batch*head, layer): fp32 column sums of K for each 32-token
 //                   half, and all of V's quantisation -- V is read once. A block's V scales are powers of two, one per
 //                   (key group, channel): group g is the block's 32-token half g, the K-block g of the attention's
@@ -14,6 +14,8 @@
 //                   32 g + c % 32 and selects byte c / 32).
 //   2. kv_finalize: per (batch*head, layer, 16 channels), the half-block sums added into blocks and 4-block
 //                   super-blocks in parallel, the super-blocks left to right, then the mean in the inputs' format.
+//                   Chunks of at most 32 blocks have no such launch: every workgroup of pass 3 forms its head's mean
+//                   itself, in the same order (own_mean).
 //   3. kv_quant:    K - mean -> int8 per 64-token block (reads K a second time); with V (a caller that wrote the
 //                   K partials itself and never read V) also V as in pass 1.
 // The column-sum order is fixed (see the oracle's chunk_mean): s = x[4q] + x[4q+1] + x[4q+2] + x[4q+3] per
@@ -264,8 +266,17 @@ __global__ __launch_bounds__(256) void kv_finalize_kernel(ReqArgs a, const float
       buf[uu * FIN_CH + c] = us;
     }
     __syncthreads();
-    if (j == 0)
-      for (int uu = 0; uu < nu; ++uu) tot = __fadd_rn(tot, buf[uu * FIN_CH + c]);
+    if (j == 0) {
+      int uu = 0;   // eight reads in flight ahead of the serial additions
+      for (; uu + 8 <= nu; uu += 8) {
+        float f[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = buf[(uu + i) * FIN_CH + c];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) tot = __fadd_rn(tot, f[i]);
+      }
+      for (; uu < nu; ++uu) tot = __fadd_rn(tot, buf[uu * FIN_CH + c]);
+    }
     __syncthreads();
   }
   if (j == 0) {
@@ -274,27 +285,74 @@ __global__ __launch_bounds__(256) void kv_finalize_kernel(ReqArgs a, const float
   }
 }
 
+// A head's mean inside the quantiser, for chunks of at most OWN_MEAN_BLOCKS blocks: the finaliser's sums in its order,
+// thread (p, c) = (t >> 7, t & 127) the super-blocks u = p, p + 2, .. of channel c, all loads independent. It replaces
+// a launch of 3.6-4.8 us (and the gap before it) by at most 32 KB of L2 reads per workgroup; at the DiT's 95 blocks
+// those would be 97 KB each, 110 MB a layer, so longer chunks keep the finaliser.
+constexpr int OWN_MEAN_BLOCKS = 32;
+template <bool F16>
+__device__ __forceinline__ void own_mean(const ReqArgs& a, const float* __restrict__ bsum, float (*s_u)[D],
+                                         float* s_mean, float* __restrict__ km_out) {
+  const int c = threadIdx.x & (D - 1), p = threadIdx.x >> 7;
+  const int nsup = (int)((a.nb + REQ_SUPER - 1) / REQ_SUPER);
+  float hs[OWN_MEAN_BLOCKS / REQ_SUPER / 2][REQ_SUPER][2];
+#pragma unroll
+  for (int n = 0; n < OWN_MEAN_BLOCKS / REQ_SUPER / 2; ++n)
+#pragma unroll
+    for (int i = 0; i < REQ_SUPER; ++i) {
+      const int b = (2 * n + p) * REQ_SUPER + i;
+      const bool ok = b < a.nb;
+      const float* src = bsum + (int64_t)(ok ? b : 0) * 2 * D + c;
+      hs[n][i][0] = ok ? src[0] : 0.f;
+      hs[n][i][1] = ok ? src[D] : 0.f;
+    }
+#pragma unroll
+  for (int n = 0; n < OWN_MEAN_BLOCKS / REQ_SUPER / 2; ++n) {
+    float us = 0.f;   // absent blocks add +0, as in the finaliser
+#pragma unroll
+    for (int i = 0; i < REQ_SUPER; ++i) us = __fadd_rn(us, __fadd_rn(hs[n][i][0], hs[n][i][1]));
+    s_u[2 * n + p][c] = us;
+  }
+  __syncthreads();
+  if (p == 0) {
+    float f[OWN_MEAN_BLOCKS / REQ_SUPER], tot = 0.f;
+#pragma unroll
+    for (int u = 0; u < OWN_MEAN_BLOCKS / REQ_SUPER; ++u) f[u] = s_u[u][c];
+#pragma unroll
+    for (int u = 0; u < OWN_MEAN_BLOCKS / REQ_SUPER; ++u)
+      if (u < nsup) tot = __fadd_rn(tot, f[u]);
+    const float mean = round16<F16>(__fdiv_rn(tot, (float)a.len));
+    s_mean[c] = mean;
+    if (km_out) km_out[c] = mean;
+  }
+  __syncthreads();
+}
+
 // Thread t owns channels 8*(t & 15) .. +8 and the 4 consecutive keys 4*(t >> 4) .. +4 of the block. Layers go last
 // to first: the statistics pass read the last layers most recently, so the first re-reads can still find them in
-// the memory-side cache. WITH_V: V of the block is quantised here too.
-template <bool F16, bool WITH_V>
+// the memory-side cache. WITH_V: V of the block is quantised here too. OWN: the mean is formed here from part_sum
+// and written to km by the head's first block; otherwise read from km.
+template <bool F16, bool WITH_V, bool OWN>
 __global__ __launch_bounds__(256) void kv_quant_kernel(const uint16_t* __restrict__ k,
                                                        const uint16_t* __restrict__ v, ReqArgs a,
+                                                       const float* __restrict__ part_sum,
                                                        int8_t* __restrict__ k8, float* __restrict__ k_scale,
-                                                       const float* __restrict__ km, uint8_t* __restrict__ v8,
+                                                       float* __restrict__ km, uint8_t* __restrict__ v8,
                                                        uint8_t* __restrict__ v8lo, uint8_t* __restrict__ v_scale) {
   __shared__ float s_red[4];
   __shared__ std::conditional_t<WITH_V, VBlockLds, int> s_v;   // (no V tile without V)
+  __shared__ float s_u[OWN ? OWN_MEAN_BLOCKS / REQ_SUPER : 1][D];
+  __shared__ __attribute__((aligned(16))) float s_mean[D];
   const int blk = blockIdx.x, bh = blockIdx.y, layer = gridDim.z - 1 - blockIdx.z;
   const int t = threadIdx.x, cg = t & 15, kq = t >> 4;
   const int64_t b = bh / a.heads, h = bh % a.heads;
   const uint16_t* kp = k + layer * a.k_sl + b * a.k_sb + h * a.k_sh + cg * 8;
   const int64_t slot_bh = ((int64_t)layer * a.slots + a.slot) * a.bh + bh;
-  float mean[8];
-  {
-    const float* kmp = km + slot_bh * D + cg * 8;
+  v4i kw[4];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) mean[c] = kmp[c];
+  for (int j = 0; j < 4; ++j) {
+    const int64_t tok = (int64_t)blk * KB + kq * 4 + j;
+    kw[j] = tok < a.len ? *(const v4i*)(kp + tok * a.k_st) : v4i{0, 0, 0, 0};
   }
   v4i vw[4];
   if constexpr (WITH_V) {
@@ -305,15 +363,25 @@ __global__ __launch_bounds__(256) void kv_quant_kernel(const uint16_t* __restric
       vw[j] = tok < a.len ? *(const v4i*)(vp + tok * a.v_st) : v4i{0, 0, 0, 0};
     }
   }
+  float mean[8];
+  {
+    const float* kmp = km + slot_bh * D + cg * 8;
+    if constexpr (OWN) {
+      own_mean<F16>(a, part_sum + ((int64_t)layer * a.bh + bh) * a.nb * 2 * D, s_u, s_mean,
+                    blk == 0 ? km + slot_bh * D : nullptr);
+      kmp = s_mean + cg * 8;
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) mean[c] = kmp[c];
+  }
   float x[4][8];
   float amax = 0.f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int64_t tok = (int64_t)blk * KB + kq * 4 + j;
     const bool ok = tok < a.len;
-    v4i kw = ok ? *(const v4i*)(kp + tok * a.k_st) : v4i{0, 0, 0, 0};
     float kf[8];
-    unpack8t<F16>(kw, kf);
+    unpack8t<F16>(kw[j], kf);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       x[j][c] = ok ? __fsub_rn(kf[c], mean[c]) : 0.f;
@@ -385,29 +453,20 @@ int kv_requant_launch(bool with_stats, bool f16, const uint16_t* k, const uint16
   if (const int dv = check_device()) return dv;
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)a.nb, (unsigned)a.bh, (unsigned)layers);
-  const dim3 fgrid((unsigned)a.bh, (unsigned)layers, D / FIN_CH);
-  // with the statistics pass, V is quantised there and the last pass is K only; without it, the last pass does both
-  if (f16) {
+  const dim3 fgrid((unsigned)a.bh, (unsigned)layers, D / FIN_CH), block(256);
+  const bool own = a.nb <= OWN_MEAN_BLOCKS;
+  const auto run = [&](auto f16c) {
+    constexpr bool F16 = decltype(f16c)::value;
+    // with the statistics pass, V is quantised there and the last pass is K only; without it, the last pass does both
     if (with_stats)
-      hipLaunchKernelGGL(kv_stats_kernel<true>, grid, dim3(256), 0, st, k, v, a, part_sum, v8, v8lo, v_scale);
-    hipLaunchKernelGGL(kv_finalize_kernel<true>, fgrid, dim3(256), 0, st, a, part_sum, km);
-    if (with_stats)
-      hipLaunchKernelGGL((kv_quant_kernel<true, false>), grid, dim3(256), 0, st, k, v, a, k8, k_scale, km, v8, v8lo,
-                         v_scale);
-    else
-      hipLaunchKernelGGL((kv_quant_kernel<true, true>), grid, dim3(256), 0, st, k, v, a, k8, k_scale, km, v8, v8lo,
-                         v_scale);
-  } else {
-    if (with_stats)
-      hipLaunchKernelGGL(kv_stats_kernel<false>, grid, dim3(256), 0, st, k, v, a, part_sum, v8, v8lo, v_scale);
-    hipLaunchKernelGGL(kv_finalize_kernel<false>, fgrid, dim3(256), 0, st, a, part_sum, km);
-    if (with_stats)
-      hipLaunchKernelGGL((kv_quant_kernel<false, false>), grid, dim3(256), 0, st, k, v, a, k8, k_scale, km, v8, v8lo,
-                         v_scale);
-    else
-      hipLaunchKernelGGL((kv_quant_kernel<false, true>), grid, dim3(256), 0, st, k, v, a, k8, k_scale, km, v8, v8lo,
-                         v_scale);
-  }
+      hipLaunchKernelGGL(kv_stats_kernel<F16>, grid, block, 0, st, k, v, a, part_sum, v8, v8lo, v_scale);
+    if (!own) hipLaunchKernelGGL(kv_finalize_kernel<F16>, fgrid, block, 0, st, a, part_sum, km);
+    const auto quant = with_stats ? (own ? kv_quant_kernel<F16, false, true> : kv_quant_kernel<F16, false, false>)
+                                  : (own ? kv_quant_kernel<F16, true, true> : kv_quant_kernel<F16, true, false>);
+    hipLaunchKernelGGL(quant, grid, block, 0, st, k, v, a, part_sum, k8, k_scale, km, v8, v8lo, v_scale);
+  };
+  if (f16) run(std::true_type{});
+  else run(std::false_type{});
   if (hipGetLastError() != hipSuccess) return LBW_E_LAUNCH;
   return LBW_OK;
 }
