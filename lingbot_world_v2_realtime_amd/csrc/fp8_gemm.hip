@@ -35,6 +35,7 @@ struct GemmArgs {
   const uint16_t* bias;  // bf16 [n] or null
   uint16_t* out;         // bf16 [m][n]
   int m, n, k, mt, nt;   // mt x nt tiles
+  int first, tiles;      // the tiles of this launch: first .. first + tiles of the tile order
 };
 
 // The last stage of a K that is not a multiple of 128 reads its missing 16-byte chunks from here.
@@ -449,28 +450,38 @@ struct Gemm {
 };
 
 // Tile order: 4 token tiles for each channel tile, so the tiles an XCD works on at a time share few operand rows.
+// HALF: mt x nt are tiles twice as wide, each two tiles in a row of this order.
+template <bool HALF>
 __device__ __forceinline__ void tile_at(const GemmArgs& a, int id, int& tm, int& tn) {
+  const int sub = HALF ? id & 1 : 0;
+  if (HALF) id >>= 1;
   constexpr int GM = 4;
   const int grp = id / (GM * a.nt), first = grp * GM, gm = a.mt - first < GM ? a.mt - first : GM;
   const int in = id - grp * GM * a.nt;
   tm = first + in % gm;
-  tn = in / gm;
+  tn = HALF ? 2 * (in / gm) + sub : in / gm;
 }
 
 // Persistent: workgroup g runs on XCD g % 8, each XCD takes a contiguous range of the tiles, dealt round-robin among
 // its workgroups. AHEAD: the next tile's parameters and first stages are loaded while this one is finished and stored.
-template <int TM, int TN, int WGM, int WGN, int NST, int KS, bool AHEAD, bool MX>
+template <int TM, int TN, int WGM, int WGN, int NST, int KS, bool AHEAD, bool HALF, bool MX>
 __global__ __launch_bounds__(64 * WGM * WGN * KS, (Gemm<TM, TN, WGM, WGN, NST, KS, AHEAD, MX>::WAVES))
 void gemm_kernel(GemmArgs a) {
   using G = Gemm<TM, TN, WGM, WGN, NST, KS, AHEAD, MX>;
   static_assert(KS == 1 || !AHEAD, "the shares are added in the stages");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[G::LDS];
-  const int tiles = a.mt * a.nt, x = blockIdx.x & 7, gx = gridDim.x >> 3;
-  const int lo = (int)((int64_t)x * tiles / 8), hi = (int)((int64_t)(x + 1) * tiles / 8);
+  const int x = blockIdx.x & 7, gx = gridDim.x >> 3;
+  const int lo = a.first + (int)((int64_t)x * a.tiles / 8), hi = a.first + (int)((int64_t)(x + 1) * a.tiles / 8);
   int id = lo + (blockIdx.x >> 3), tm, tn;
-  if (id >= hi) return;
+  const auto seek = [&]() {   // the tile of id, passing over halves past the last channel; false at the range's end
+    for (; id < hi; id += gx) {
+      tile_at<HALF>(a, id, tm, tn);
+      if (!HALF || tn * TN < a.n) return true;
+    }
+    return false;
+  };
+  if (!seek()) return;
   G g(a, lds);
-  tile_at(a, id, tm, tn);
   int par = 0;
   g.begin(tm, tn, 0);
   bool pend = false;
@@ -479,12 +490,9 @@ void gemm_kernel(GemmArgs a) {
     g.sum(acc, pend);
     const int m0 = g.m0, n0 = g.n0;
     id += gx;
-    const bool more = id < hi, mine = g.gather(acc);
+    const bool more = seek(), mine = g.gather(acc);
     stage_barrier();   // every wave has read its last fragments (or the other share's sums)
-    if (AHEAD && more) {
-      tile_at(a, id, tm, tn);
-      g.begin(tm, tn, par ^ 1);
-    }
+    if (AHEAD && more) g.begin(tm, tn, par ^ 1);
     const bool full = m0 + TM <= a.m && n0 + TN <= a.n;
     if (mine) {
       if (full) g.template finish<true>(acc, m0, n0, par);
@@ -497,20 +505,24 @@ void gemm_kernel(GemmArgs a) {
       par ^= 1;
     } else {
       stage_barrier();   // every wave has read its results back
-      tile_at(a, id, tm, tn);
       g.begin(tm, tn, 0);
     }
   }
 }
 
-template <int TM, int TN, int WGM, int WGN, int NST, int KS, bool AHEAD, bool MX>
-static void gemm_launch(GemmArgs& a, hipStream_t stream) {
+// Tiles [first, first + tiles) of a's order (all of them when tiles is 0). HALF: a.mt, a.nt are set by the caller.
+template <int TM, int TN, int WGM, int WGN, int NST, int KS, bool AHEAD, bool HALF, bool MX>
+static void gemm_launch(GemmArgs& a, hipStream_t stream, int64_t first = 0, int64_t tiles = 0) {
   using G = Gemm<TM, TN, WGM, WGN, NST, KS, AHEAD, MX>;
-  a.mt = (a.m + TM - 1) / TM;
-  a.nt = (a.n + TN - 1) / TN;
-  const int64_t per = ((int64_t)a.mt * a.nt + 7) / 8, cap = 32 * (163840 / G::LDS);
-  hipLaunchKernelGGL((gemm_kernel<TM, TN, WGM, WGN, NST, KS, AHEAD, MX>), dim3((unsigned)(8 * (per < cap ? per : cap))),
-                     dim3(G::THREADS), 0, stream, a);
+  if (!HALF) {
+    a.mt = (a.m + TM - 1) / TM;
+    a.nt = (a.n + TN - 1) / TN;
+  }
+  a.first = (int)first;
+  a.tiles = (int)(tiles ? tiles : (int64_t)a.mt * a.nt);
+  const int64_t per = ((int64_t)a.tiles + 7) / 8, cap = 32 * (163840 / G::LDS);
+  hipLaunchKernelGGL((gemm_kernel<TM, TN, WGM, WGN, NST, KS, AHEAD, HALF, MX>),
+                     dim3((unsigned)(8 * (per < cap ? per : cap))), dim3(G::THREADS), 0, stream, a);
 }
 
 // The tile for a shape, by tile counts (one workgroup per CU but for the 64 x 64 form: 256 CUs). Measured in us at
@@ -529,20 +541,32 @@ static void gemm_launch(GemmArgs& a, hipStream_t stream) {
 // rounds x (stages x time of a stage + fixed part) as fitted to these figures. The MX form of 256 x 256 does not fit
 // the registers beside its scales (29.3 us against 29.3 for 192 x 192 at 1508 x 1536 x 8960, 114 against 102 at 6032
 // tokens), so MX stops at 192 x 192.
+// A last round of at most 128 such tiles goes out as half tiles in a launch of its own, which takes about half a
+// round (a half past the last channel is passed over): feed-forward at 6032 tokens 197.8 -> 192.0 us. (In the same launch,
+// after the whole tiles, the second tile body cost 28 spilled registers and 7 us.)
 template <bool MX>
 static int gemm_dispatch(GemmArgs& a, hipStream_t stream) {
   const auto tiles = [&](int64_t t) { return ((a.m + t - 1) / t) * ((a.n + t - 1) / t); };
   const auto rounds = [&](int64_t t) { return (tiles(t) + 255) / 256; };
-  const int64_t ns = (a.k + GK - 1) / GK;
+  const int64_t ns = (a.k + GK - 1) / GK, all = tiles(256), rest = all % 256;
+  const bool halves = all > 256 && rest > 0 && rest <= 128;
+  const int64_t half_rounds = all / 256 * 2 + (rest == 0 ? 0 : halves ? 1 : 2);
   if (tiles(64) <= 256) {
-    if (a.k >= 4096) gemm_launch<64, 64, 2, 2, 4, 2, false, MX>(a, stream);
-    else gemm_launch<64, 64, 2, 2, 4, 1, false, MX>(a, stream);
+    if (a.k >= 4096) gemm_launch<64, 64, 2, 2, 4, 2, false, false, MX>(a, stream);
+    else gemm_launch<64, 64, 2, 2, 4, 1, false, false, MX>(a, stream);
   } else if (tiles(128) <= 256) {
-    gemm_launch<128, 128, 4, 2, 4, 1, false, MX>(a, stream);
-  } else if (MX || rounds(192) == 1 || rounds(192) * (82 * ns + 700) <= rounds(256) * (100 * ns + 1100)) {
-    gemm_launch<192, 192, 2, 6, 3, 1, false, MX>(a, stream);
+    gemm_launch<128, 128, 4, 2, 4, 1, false, false, MX>(a, stream);
+  } else if (MX || rounds(192) == 1 || rounds(192) * (82 * ns + 700) <= half_rounds * (50 * ns + 550)) {
+    gemm_launch<192, 192, 2, 6, 3, 1, false, false, MX>(a, stream);
   } else {
-    if constexpr (!MX) gemm_launch<256, 256, 4, 2, 2, 1, true, false>(a, stream);
+    if constexpr (!MX) {
+      if (halves) {
+        gemm_launch<256, 256, 4, 2, 2, 1, true, false, false>(a, stream, 0, all - rest);
+        gemm_launch<256, 128, 4, 2, 3, 1, false, true, false>(a, stream, 2 * (all - rest), 2 * rest);
+      } else {
+        gemm_launch<256, 256, 4, 2, 2, 1, true, false, false>(a, stream);
+      }
+    }
   }
   if (hipGetLastError() != hipSuccess) return LBW_E_LAUNCH;
   return LBW_OK;
