@@ -41,7 +41,9 @@ struct ProArgs {
   int seg_slot[LBW_MAX_SEGMENTS];
 };
 
-// (cos, sin) of rows row0 .. row0 + 31 into LDS, [row][pair]; rows past len get (1, 0).
+// (cos, sin) of rows row0 .. row0 + 31 into LDS, [row][pair & 3][pair >> 2]; rows past len get (1, 0). Lane g of a row
+// reads pairs 4 g + q, so for each q the 16 lanes read 256 contiguous bytes (in pair order they were 64 bytes apart:
+// four lanes to a bank group).
 __device__ __forceinline__ void stage_rope(double2* s_cs, const double2* __restrict__ tab, const ProArgs& a,
                                            int64_t row0) {
   for (int i = threadIdx.x; i < PR * RP; i += blockDim.x) {
@@ -54,7 +56,7 @@ __device__ __forceinline__ void stage_rope(double2* s_cs, const double2* __restr
       const uint32_t row = j < RS0 ? (uint32_t)a.start_frame + f : (j < RS1 ? rem / gw : rem % gw);
       cs = tab[row * RP + j];
     }
-    s_cs[i] = cs;
+    s_cs[r * RP + (j & 3) * (RP / 4) + (j >> 2)] = cs;
   }
 }
 
@@ -105,6 +107,7 @@ __device__ __forceinline__ void norm_rope_rows(uint32_t (&x)[2][4][4], const uin
                                                const ProArgs& a, int64_t row0, double* s_ss, float* s_r,
                                                const double2* s_cs) {
   const int lane = threadIdx.x & 63, h = threadIdx.x >> 6, rq = lane >> 4, g = lane & 15;
+  const v4i wv = *(const v4i*)(w + h * D + g * 8);   // in flight with the rows, not after the barriers below
   double ss[2][4];
 #pragma unroll
   for (int s = 0; s < 2; ++s)
@@ -113,9 +116,10 @@ __device__ __forceinline__ void norm_rope_rows(uint32_t (&x)[2][4][4], const uin
       double acc = 0.0;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
+        // (a bf16 square has 16 bits, so the FMA adds the same exact product as a multiply and an add would)
         const double x0 = (double)bf_lo(x[s][j][q]), x1 = (double)bf_hi(x[s][j][q]);
-        acc = acc + x0 * x0;
-        acc = acc + x1 * x1;
+        acc = __builtin_fma(x0, x0, acc);
+        acc = __builtin_fma(x1, x1, acc);
       }
       ss[s][j] = acc;
     }
@@ -130,27 +134,30 @@ __device__ __forceinline__ void norm_rope_rows(uint32_t (&x)[2][4][4], const uin
       for (int j = 0; j < 4; ++j) s_ss[(4 * (rq + 4 * s) + j) * PRO_MAX_HEADS + h] = ss[s][j];
   __syncthreads();
   if (threadIdx.x < PR) {   // one thread per row: the heads' partials in order, and the row's scale
-    double tot = 0.0;
-    for (int hh = 0; hh < a.heads; ++hh) tot = tot + s_ss[threadIdx.x * PRO_MAX_HEADS + hh];
+    double p[PRO_MAX_HEADS], tot = 0.0;   // all reads first: one by one, each addition waits for an LDS round trip
+#pragma unroll
+    for (int hh = 0; hh < PRO_MAX_HEADS; ++hh) p[hh] = s_ss[threadIdx.x * PRO_MAX_HEADS + hh];
+#pragma unroll
+    for (int hh = 0; hh < PRO_MAX_HEADS; ++hh)
+      if (hh < a.heads) tot = tot + p[hh];
     const float ms = (float)(tot / (double)(a.heads * D));
     s_r[threadIdx.x] = row0 + threadIdx.x < a.len ? (float)(1.0 / sqrt((double)(ms + a.eps))) : 0.f;
   }
   __syncthreads();
-  const v4i wv = *(const v4i*)(w + h * D + g * 8);
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int row = 4 * (rq + 4 * s) + j;
       const float r = s_r[row];
-      const double2* cs = s_cs + row * RP + g * 4;
+      const double2* cs = s_cs + row * RP + g;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const uint32_t u = x[s][j][q], wq = (uint32_t)wv[q];
         const uint32_t y = bf_pair(bf_lo(u) * r, bf_hi(u) * r);                     // bf16(x r)
         const uint32_t nn = bf_pair(bf_lo(y) * bf_lo(wq), bf_hi(y) * bf_hi(wq));    // bf16(y w)
         const float n0 = bf_lo(nn), n1 = bf_hi(nn);
-        const double2 c = cs[q];
+        const double2 c = cs[q * (RP / 4)];
         const double re = (double)n0 * c.x - (double)n1 * c.y;
         const double im = (double)n0 * c.y + (double)n1 * c.x;
         x[s][j][q] = bf_pair((float)re, (float)im);
