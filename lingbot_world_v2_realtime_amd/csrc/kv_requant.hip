@@ -12,7 +12,7 @@
 //                   set), and the block's 256-byte E8M0 table (byte (32 g + c % 32) * 4 + c / 32 = 127 + e of
 //                   channel c, group g: the attention lane that scales channel c's row for group g reads dword
 //                   32 g + c % 32 and selects byte c / 32).
-//   2. kv_finalize: per (batch*head, layer, 16 channels), the half-block sums added into blocks and 4-block
+//   2. kv_finalize: per (batch*head, layer, 16 or 32 channels), the half-block sums added into blocks and 4-block
 //                   super-blocks in parallel, the super-blocks left to right, then the mean in the inputs' format.
 //                   Chunks of at most 32 blocks have no such launch: every workgroup of pass 3 forms its head's mean
 //                   itself, in the same order (own_mean).
@@ -237,14 +237,16 @@ __global__ __launch_bounds__(256) void kv_stats_kernel(const uint16_t* __restric
   vblock_store(s_v, v8, v8lo, v_scale, tile);
 }
 
-// One workgroup per (batch*head, layer, group of 16 channels). Thread (j, c) = (t >> 4, t & 15) forms the
-// super-block sums U[u] = B[4u] + .. + B[4u+3] of channel 16 cgrp + c for u = j, j + 16, .. (all of them at
-// once, in parallel); then one thread per channel sums the U left to right.
-constexpr int FIN_CH = 16;                 // channels per finaliser workgroup
-constexpr int FIN_J = 256 / FIN_CH;        // super-block lanes per channel
-template <bool F16>
+// One workgroup per (batch*head, layer, group of CH channels). Thread (j, c) = (t / CH, t % CH) forms the
+// super-block sums U[u] = B[4u] + .. + B[4u+3] of channel CH cgrp + c for u = j, j + 256 / CH, .. (all of them at
+// once, in parallel); then one thread per channel sums the U left to right. CH = 32 reads whole 128-byte lines (30
+// layers: 14.6 -> 12.2 us); 16 has twice the threads on a channel's loads, which counts when the grid is small (one
+// layer of 12 heads: 4.8 against 6.1 us). The host takes 32 from 2 workgroups a CU on.
+constexpr int64_t FIN_WIDE = 512;
+template <bool F16, int FIN_CH>
 __global__ __launch_bounds__(256) void kv_finalize_kernel(ReqArgs a, const float* __restrict__ part_sum,
                                                           float* __restrict__ km) {
+  constexpr int FIN_J = 256 / FIN_CH;   // super-block lanes per channel
   __shared__ float buf[FIN_U * FIN_J * FIN_CH];
   const int bh = blockIdx.x, layer = blockIdx.y, cgrp = blockIdx.z;
   const int t = threadIdx.x, c = t & (FIN_CH - 1), j = t / FIN_CH, ch = cgrp * FIN_CH + c;
@@ -453,14 +455,18 @@ int kv_requant_launch(bool with_stats, bool f16, const uint16_t* k, const uint16
   if (const int dv = check_device()) return dv;
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)a.nb, (unsigned)a.bh, (unsigned)layers);
-  const dim3 fgrid((unsigned)a.bh, (unsigned)layers, D / FIN_CH), block(256);
+  const dim3 block(256);
   const bool own = a.nb <= OWN_MEAN_BLOCKS;
   const auto run = [&](auto f16c) {
     constexpr bool F16 = decltype(f16c)::value;
     // with the statistics pass, V is quantised there and the last pass is K only; without it, the last pass does both
     if (with_stats)
       hipLaunchKernelGGL(kv_stats_kernel<F16>, grid, block, 0, st, k, v, a, part_sum, v8, v8lo, v_scale);
-    if (!own) hipLaunchKernelGGL(kv_finalize_kernel<F16>, fgrid, block, 0, st, a, part_sum, km);
+    if (!own) {
+      const int ch = a.bh * layers * (D / 32) >= FIN_WIDE ? 32 : 16;
+      const auto fin = ch == 32 ? kv_finalize_kernel<F16, 32> : kv_finalize_kernel<F16, 16>;
+      hipLaunchKernelGGL(fin, dim3((unsigned)a.bh, (unsigned)layers, (unsigned)(D / ch)), block, 0, st, a, part_sum, km);
+    }
     const auto quant = with_stats ? (own ? kv_quant_kernel<F16, false, true> : kv_quant_kernel<F16, false, false>)
                                   : (own ? kv_quant_kernel<F16, true, true> : kv_quant_kernel<F16, true, false>);
     hipLaunchKernelGGL(quant, grid, block, 0, st, k, v, a, part_sum, k8, k_scale, km, v8, v8lo, v_scale);
