@@ -503,8 +503,7 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a, const int8_t* __
       if (FAST || it + LEAD < n) {   // steady state as one constant wait (a general count is a chain of branches)
         wait_vm(NPB * (LEAD - 1));
       } else {
-        const int ahead = n - 1 - (it + 1);
-        wait_vm(ahead > 0 ? NPB * ahead : 0);
+        wait_vm(0);   // no more loads are issued: the exact count saves less than its chain of branches costs
       }
     }
     phase_barrier();
@@ -600,8 +599,7 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a, const int8_t* __
       if (FAST || it + LEAD < n) {   // steady state as one constant wait (a general count is a chain of branches)
         wait_vm(NPB * (LEAD - 1));
       } else {
-        const int ahead = n - 1 - (it + 1);
-        wait_vm(ahead > 0 ? NPB * ahead : 0);
+        wait_vm(0);   // no more loads are issued: the exact count saves less than its chain of branches costs
       }
     }
     phase_barrier();
@@ -670,6 +668,15 @@ __device__ __forceinline__ void store_part(const Piece& st, float* __restrict__ 
   if (g == 0) *(float2*)(ml_part + (slot_idx * QT + row) * 2) = make_float2(st.m, st.l);
 }
 
+// Every 64-byte line of the arguments into the scalar cache at once. They are read where they are needed, most behind
+// a computed index or a branch, and each first read of a line is a ~0.4 us miss: one after another they were 2 us of a
+// workgroup's start (cycle stamps; a short call's workgroup lives ~8 us).
+__device__ __forceinline__ void touch_args(const AttnArgs& a) {
+  asm volatile("" ::"s"(a.lq), "s"(a.nbc), "s"(a.sl2), "s"(a.seg_slot[0]), "s"(a.seg_fb[0]), "s"(a.seg_lead[0]),
+               "s"(a.seg_span[0]), "s"(a.seg_blk0[0]), "s"(a.split0[0]), "s"(a.t_lo[0]), "s"(a.ts[0]), "s"(a.uq[0]),
+               "s"(a.ur[0]), "s"(a.inv_gx));
+}
+
 template <bool TWO, bool LOGITS>
 __global__ __launch_bounds__(AT_THREADS, 1) void attn_fwd_kernel(const int8_t* __restrict__ q8,
                                                                  const float* __restrict__ q_scale,
@@ -683,6 +690,7 @@ __global__ __launch_bounds__(AT_THREADS, 1) void attn_fwd_kernel(const int8_t* _
                                                                  float* __restrict__ ml_part, int32_t* __restrict__ logits,
                                                                  AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[AT_LDS];
+  touch_args(a);
   const int gid = blockIdx.x, x = gid % XCDS, i = gid / XCDS;
   const int w = threadIdx.x >> 6;
   // whole tiles, dealt round-robin among this XCD's workgroups, then this workgroup's piece of the split tiles: one
@@ -726,6 +734,7 @@ constexpr int MERGE_N = 4;
 __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict__ o_part,
                                                          const float* __restrict__ ml_part,
                                                          uint16_t* __restrict__ out, AttnArgs a) {
+  touch_args(a);
   const int st = blockIdx.x / MERGE_WGS, w = blockIdx.x / 4 % AT_WAVES, mt = blockIdx.x & 3;
   int x = 0;
   while (x + 1 < XCDS && st >= a.split0[x + 1]) ++x;
