@@ -383,8 +383,11 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a, const int8_t* __
   // most passes: the loader's block it + LEAD exists and lies in the loader's current chunk, and block it is
   // neither the first nor the last block of its chunk (so no new logit bias, no key mask, no chunk step). It
   // returns true after the last MFMA phase (it == n).
-  auto pass = [&](auto fast) -> bool {
-    constexpr bool FAST = decltype(fast)::value;
+  // MODE 1 is that form, MODE 0 the general one. MODE 2 is the fast form of a piece's last blocks: no block left to
+  // load, otherwise as MODE 1.
+  auto pass = [&](auto mode) -> bool {
+    constexpr int MODE = decltype(mode)::value;
+    constexpr bool FAST = MODE != 0;
     // ---- MFMA phase: S of block it, P V of block it - 1 ----
     // (wave priorities stay equal: raising this phase's cost 0.3 % of kernel time, raising the softmax phase's 0.2 %)
     // LDS reads run ahead of the MFMAs that consume them: all eight K fragments and the first two V fragments
@@ -457,9 +460,9 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a, const int8_t* __
     // phase, where the wave mostly waits for the matrix core (the softmax phase slows down with it), and after
     // the first two QK MFMAs, so the matrix core starts at once and the issue hides under their execution
     // (-1 to -2 % against issuing it before them, same-box A/B)
-    if (FAST || it + LEAD < n) {
+    if (MODE == 1 || (MODE == 0 && it + LEAD < n)) {
       issue(ldstage);
-      advance(fast);
+      advance(std::bool_constant<MODE == 1>{});
       ldstage = ldstage + 1 == NSTAGE ? 0 : ldstage + 1;
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -500,7 +503,7 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a, const int8_t* __
     // form waits in both groups (no branch): A's pieces of block it + 1 were issued LEAD - 1 passes ago, and A
     // needs them by the end of this pass anyway.
     if (FAST || !grp_a) {
-      if (FAST || it + LEAD < n) {   // steady state as one constant wait (a general count is a chain of branches)
+      if (MODE == 1 || (MODE == 0 && it + LEAD < n)) {   // steady state as one constant wait (a general count is a chain of branches)
         wait_vm(NPB * (LEAD - 1));
       } else {
         wait_vm(0);   // no more loads are issued: the exact count saves less than its chain of branches costs
@@ -596,7 +599,7 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a, const int8_t* __
       lead = a.seg_lead[c];
     }
     if (FAST || grp_a) {   // A's pieces of block it + 1 have landed (blocks up to it + LEAD may still be in flight)
-      if (FAST || it + LEAD < n) {   // steady state as one constant wait (a general count is a chain of branches)
+      if (MODE == 1 || (MODE == 0 && it + LEAD < n)) {   // steady state as one constant wait (a general count is a chain of branches)
         wait_vm(NPB * (LEAD - 1));
       } else {
         wait_vm(0);   // no more loads are issued: the exact count saves less than its chain of branches costs
@@ -616,12 +619,20 @@ __device__ __forceinline__ void attend_range(const AttnArgs& a, const int8_t* __
     if (n - LEAD - it < f) f = n - LEAD - it;
     if (c != c_prev || lead > 0) f = 0;
     if (f > 0) {
-      for (int i = 0; i < f; ++i) pass(std::true_type{});
+      for (int i = 0; i < f; ++i) pass(std::integral_constant<int, 1>{});
       it += f;
       lrem -= f;
       crem -= f;
     }
-    if (pass(std::false_type{})) break;
+    // and those of the piece's last blocks that are not their chunk's first or last
+    f = crem - 1 < n - it ? crem - 1 : n - it;
+    if (it + LEAD < n || c != c_prev || lead > 0) f = 0;
+    if (f > 0) {
+      for (int i = 0; i < f; ++i) pass(std::integral_constant<int, 2>{});
+      it += f;
+      crem -= f;
+    }
+    if (pass(std::integral_constant<int, 0>{})) break;
   }
   if (grp_a) phase_barrier();   // matches group B's extra barrier at the start
   phase_barrier();               // every wave is done with the stages before they are refilled
