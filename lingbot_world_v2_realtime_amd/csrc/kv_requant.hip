@@ -405,12 +405,8 @@ __global__ __launch_bounds__(256) void kv_quant_kernel(const uint16_t* __restric
   int8_t* kout = k8 + (slot_bh * a.cap + (int64_t)blk * KB) * D + cg * 8;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      lo |= ((uint32_t)quant_i8(x[j][c], recip) & 0xFFu) << (8 * c);
-      hi |= ((uint32_t)quant_i8(x[j][c + 4], recip) & 0xFFu) << (8 * c);
-    }
+    const uint32_t lo = quant4_i8(x[j][0], x[j][1], x[j][2], x[j][3], recip);
+    const uint32_t hi = quant4_i8(x[j][4], x[j][5], x[j][6], x[j][7], recip);
     store_once(kout + (kq * 4 + j) * D, v2i{(int)lo, (int)hi});
   }
   if constexpr (WITH_V) {

@@ -108,11 +108,19 @@ __device__ __forceinline__ float round16(float x) {
   else return bf16_round(x);
 }
 
-// round(x * recip) to int8 with saturation; explicit roundings so no FMA contraction can occur.
-__device__ __forceinline__ int quant_i8(float x, float recip) {
-  float r = rintf(__fmul_rn(x, recip));
-  r = fminf(fmaxf(r, -128.f), 127.f);
-  return (int)r;
+// Four values as int8 bytes, x0 lowest: round(x * recip), ties to even, saturating (a NaN gives -128, as a clamp by
+// fminf / fmaxf would). The product is rounded by itself (no FMA contraction: v_med3 stands between), the clamp to the
+// integer bounds commutes with the rounding, and adding 1.5 * 2^23 rounds to an integer whose two's complement byte is
+// the sum's lowest: three operations a value and three to pack four, against seven a value for rint, clamp, convert,
+// mask and shift. The Q quantisers are bound by their vector work once their rows are in: 6032 x 12 heads, fused prologue
+// 14.85 -> 14.32 us, quant_q 6.61 -> 5.96 us, one-layer re-quant 18.67 -> 18.31 us.
+__device__ __forceinline__ uint32_t quant4_i8(float x0, float x1, float x2, float x3, float recip) {
+  const float x[4] = {x0, x1, x2, x3};
+  uint32_t u[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    u[i] = __float_as_uint(__fadd_rn(__builtin_amdgcn_fmed3f(__fmul_rn(x[i], recip), -128.f, 127.f), 12582912.f));
+  return __builtin_amdgcn_perm(u[1], u[0], 0x0C0C0400u) | __builtin_amdgcn_perm(u[3], u[2], 0x04000C0Cu);
 }
 
 // Cross-lane reads by DPP, within rows of 16 lanes: a VALU operand modifier, with no LDS round trip (a shuffle

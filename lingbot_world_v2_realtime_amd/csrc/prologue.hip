@@ -208,9 +208,7 @@ __global__ __launch_bounds__(MAXT) void norm_rope_q_kernel(const uint16_t* __res
 #pragma unroll
       for (int hw = 0; hw < 2; ++hw) {
         const uint32_t u0 = x[s][j][2 * hw], u1 = x[s][j][2 * hw + 1];
-        wd[hw] = ((uint32_t)quant_i8(bf_lo(u0), recip) & 0xFFu) | (((uint32_t)quant_i8(bf_hi(u0), recip) & 0xFFu) << 8) |
-                 (((uint32_t)quant_i8(bf_lo(u1), recip) & 0xFFu) << 16) |
-                 (((uint32_t)quant_i8(bf_hi(u1), recip) & 0xFFu) << 24);
+        wd[hw] = quant4_i8(bf_lo(u0), bf_hi(u0), bf_lo(u1), bf_hi(u1), recip);
       }
       *(uint2*)(q8 + (bh * a.lp + t) * D + g * 8) = make_uint2(wd[0], wd[1]);
       if (q_out && t < a.len)

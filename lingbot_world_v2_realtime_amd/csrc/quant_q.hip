@@ -59,10 +59,7 @@ __global__ __launch_bounds__(64 * QQ_WAVES) void quant_q_kernel(const uint16_t* 
 #pragma unroll
       for (int hw = 0; hw < 2; ++hw) {
         const uint32_t u0 = x[s][j][2 * hw], u1 = x[s][j][2 * hw + 1];
-        wd[hw] = ((uint32_t)quant_i8(lo16<F16>(u0), recip) & 0xFFu) |
-                 (((uint32_t)quant_i8(hi16<F16>(u0), recip) & 0xFFu) << 8) |
-                 (((uint32_t)quant_i8(lo16<F16>(u1), recip) & 0xFFu) << 16) |
-                 (((uint32_t)quant_i8(hi16<F16>(u1), recip) & 0xFFu) << 24);
+        wd[hw] = quant4_i8(lo16<F16>(u0), hi16<F16>(u0), lo16<F16>(u1), hi16<F16>(u1), recip);
       }
       *(uint2*)(q8 + (bh * a.lp + t) * D + g * 8) = make_uint2(wd[0], wd[1]);
     }
