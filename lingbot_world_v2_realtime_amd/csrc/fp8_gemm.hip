@@ -3,9 +3,9 @@
 // scale per token and per output channel, applied to the finished sum) and MX (one E8M0 scale per 32 values along K
 // of each operand, applied by the MFMA itself).
 //
-// Tile: TM tokens x TN channels per workgroup, WGM x WGN waves (times KS shares of K). The W rows are the MFMA's A operand and the X rows
-// its B operand, so a lane holds one token and runs of four consecutive channels of the result. K is walked in
-// stages of 128 bytes per row (whole cache lines), streamed into NST LDS stages by direct global -> LDS loads; a
+// Tile: TM tokens x TN channels per workgroup, WGM x WGN waves (times KS shares of K). The W rows are the MFMA's A
+// operand and the X rows its B operand, so a lane holds one token and runs of four consecutive channels of the result.
+// K is walked in stages of 128 bytes per row (whole cache lines), streamed into NST LDS stages by direct global -> LDS loads; a
 // wave reads the fragments of the next 64-deep half while its matrix products run on the current one, so one barrier
 // per stage is all the synchronisation there is, and the products after it start from registers. The loads of a stage
 // are issued between the products, one after each (all at once after the barrier: 96 instead of 85 us for the 256 x
@@ -14,7 +14,7 @@
 // What bounds it: at 6032 x 8960 x 1536 the 192 x 192 tile takes 67-71 us (2.35-2.48 PFLOP/s); timing copies without
 // the loads ran 58 us, without the products 51 us, without the fragment reads 61 us, so L2 -> LDS traffic (17 TB/s
 // alone) and the matrix core (power-limited near 1.9 GHz) overlap but for ~10 us. Touching later stages in the L2
-// first, 64-byte stages in a deeper ring and half tiles in the last round were measured and brought nothing.
+// first and 64-byte stages in a deeper ring were measured and brought nothing.
 #include <type_traits>
 
 #include "../../include/lbw_gemm.h"
@@ -45,10 +45,10 @@ __device__ __forceinline__ uint32_t lds_off(const uint8_t* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p;
 }
 
-// One direct global -> LDS load of 16 bytes a lane (lane i to lds + 16 i): a uniform base plus a 32-bit byte offset
-// per lane, or a 64-bit address per lane. Inline asm, as in the attention kernel: the compiler would otherwise wait
-// for every one of them before each LDS read.
-// The wave's N pieces of one operand, STEP bytes of LDS apart: M0 is saved and restored once around them.
+// Direct global -> LDS loads of 16 bytes a lane (lane i to lds + 16 i), as inline asm like the attention kernel's: the
+// compiler would otherwise wait for every one of them before each LDS read. dma_rows: the wave's N pieces of one operand
+// from a uniform base plus a 32-bit byte offset per lane and piece, STEP bytes of LDS apart, M0 saved and restored once
+// around them (the additions to M0 write SCC). dma16_at: one piece from a 64-bit address per lane. dma4: a dword a lane.
 template <int N, int STEP>
 __device__ __forceinline__ void dma_rows(const void* base, const uint32_t* off, uint32_t lds) {
   static_assert(N >= 1 && N <= 4, "pieces");
@@ -59,17 +59,18 @@ __device__ __forceinline__ void dma_rows(const void* base, const uint32_t* off, 
     asm volatile(LBW_GEMM_HEAD "s_mov_b32 m0, %0" : "=&s"(keep) : "s"(base), "s"(lds), "v"(off[0]) : "memory");
   else if constexpr (N == 2)
     asm volatile(LBW_GEMM_HEAD LBW_GEMM_NEXT "global_load_lds_dwordx4 %5, %1\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "s"(base), "s"(lds), "v"(off[0]), "i"(STEP), "v"(off[1]) : "memory");
+                 : "=&s"(keep) : "s"(base), "s"(lds), "v"(off[0]), "i"(STEP), "v"(off[1]) : "memory", "scc");
   else if constexpr (N == 3)
     asm volatile(LBW_GEMM_HEAD LBW_GEMM_NEXT "global_load_lds_dwordx4 %5, %1\n\t" LBW_GEMM_NEXT
                  "global_load_lds_dwordx4 %6, %1\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "s"(base), "s"(lds), "v"(off[0]), "i"(STEP), "v"(off[1]), "v"(off[2]) : "memory");
+                 : "=&s"(keep) : "s"(base), "s"(lds), "v"(off[0]), "i"(STEP), "v"(off[1]), "v"(off[2])
+                 : "memory", "scc");
   else
     asm volatile(LBW_GEMM_HEAD LBW_GEMM_NEXT "global_load_lds_dwordx4 %5, %1\n\t" LBW_GEMM_NEXT
                  "global_load_lds_dwordx4 %6, %1\n\t" LBW_GEMM_NEXT "global_load_lds_dwordx4 %7, %1\n\t"
                  "s_mov_b32 m0, %0"
                  : "=&s"(keep) : "s"(base), "s"(lds), "v"(off[0]), "i"(STEP), "v"(off[1]), "v"(off[2]), "v"(off[3])
-                 : "memory");
+                 : "memory", "scc");
 #undef LBW_GEMM_NEXT
 #undef LBW_GEMM_HEAD
 }
