@@ -13,8 +13,9 @@ extern "C" {
 #endif
 
 /*
- * out[m][n] = bf16(x_scale[m] * w_scale[n] * sum_k x8[m][k] w8[n][k] + bias[n]): e4m3 operands with packed rows
- * (x8 [m][k], w8 [n][k]), fp32 sums and scales, one rounding to bf16; bias bf16 [n] or null; out [m][n] packed.
+ * out[m][n] = bf16((sum_k x8[m][k] w8[n][k] * w_scale[n]) * x_scale[m] + bias[n]): e4m3 operands with packed rows
+ * (x8 [m][k], w8 [n][k]), fp32 sums and scales, each operation in this order rounded to fp32 (as hipBLASLt's rowwise GEMM
+ * does), then one rounding to bf16; bias bf16 [n] or null; out [m][n] packed.
  * n and k multiples of 16 (n, k <= 2^22, m <= 2^30); x8, w8 and out 16-byte, the others 4-byte aligned.
  */
 int lbw_gemm_fp8_rows(const uint8_t* x8, const float* x_scale, const uint8_t* w8, const float* w_scale,

@@ -20,6 +20,8 @@
 #include "../../include/lbw_gemm.h"
 #include "lbw_common.h"
 
+#pragma clang fp contract(off)   // the epilogue's roundings are defined (without it even __fmul_rn + __fadd_rn fuse)
+
 namespace lbw {
 
 constexpr int GK = 128;             // bytes of K per stage
@@ -426,9 +428,12 @@ struct Gemm {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float v = acc[i][j][4 * q + e];
-            // MX: the sum is cut to bf16 (toward zero) before the bias is added, as the library GEMM did that ran here
-            // before and the separate addition after it: results stay what callers had
-            y[e] = MX ? __uint_as_float(__float_as_uint(v) & 0xFFFF0000u) + bi[4 * q + e] : fmaf(v * sx, sw[4 * q + e], bi[4 * q + e]);
+            // Results stay what callers had from the library GEMM that ran here before. Rowwise: the channel's scale,
+            // the token's, the bias, each operation rounded (with exact sums the same bits as hipBLASLt at every shape
+            // tried; other orders or an FMA differ in a few of 1e5 values, which FP8 layers after it amplify). MX: the
+            // sum is cut to bf16 (toward zero), then the bias added, as the separate addition did.
+            if constexpr (MX) y[e] = __uint_as_float(__float_as_uint(v) & 0xFFFF0000u) + bi[4 * q + e];
+            else y[e] = (v * sw[4 * q + e]) * sx + bi[4 * q + e];
           }
           typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
           const bf2 lo = {(__bf16)y[0], (__bf16)y[1]}, hi = {(__bf16)y[2], (__bf16)y[3]};

@@ -407,7 +407,7 @@ def _gemm_operands(x8, w8, bias):
 
 def gemm_fp8_rows(x8, x_scale, w8, w_scale, bias=None):
     """The rowwise-scaled FP8 product (lbw_gemm_fp8_rows): x8 [M, K] and w8 [N, K] float8_e4m3fn, x_scale M and w_scale
-    N fp32 values, bias bf16 [N] or None -> bf16 [M, N] = x8 w8^T x_scale w_scale + bias, rounded once."""
+    N fp32 values, bias bf16 [N] or None -> bf16 [M, N] = (x8 w8^T w_scale) x_scale + bias: fp32, in this order."""
     m, n = x8.shape[0], w8.shape[0]
     bias = _gemm_operands(x8, w8, bias)
     if x_scale.dtype != torch.float32 or w_scale.dtype != torch.float32 or x_scale.numel() != m \

@@ -62,6 +62,24 @@ def test_gemm_rows(m, k, n):
     assert (y.double() - ref).norm() <= 1.01 * (lib.double() - ref).norm()
 
 
+@pytest.mark.parametrize("m,k,n", [(65, 144, 48), (64, 8960, 1536), (1000, 272, 2048), (1509, 1536, 1536),
+                                   (2305, 128, 2320), (2048, 400, 8192), (3105, 256, 8976)])
+def test_gemm_rows_epilogue_bits(m, k, n):
+    """Operands of small integers, whose sums are exact in fp32 (|sum| <= 36 K < 2^24): what is left is the epilogue,
+    scale of the channel, scale of the token, bias, each rounded to fp32, then bf16. Every bit of it is defined."""
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    x8, w8 = (torch.randint(-6, 7, (r, k), generator=g, device=DEV).float().to(torch.float8_e4m3fn) for r in (m, n))
+    xs = torch.rand(m, 1, generator=g, device=DEV) + 0.01
+    ws = torch.rand(1, n, generator=g, device=DEV) * 1e-3 + 1e-5
+    b = (torch.randn(n, generator=g, device=DEV) * 0.1).to(torch.bfloat16)
+    v = (x8.double() @ w8.double().t()).float()
+    for bias in (None, b):
+        want = (v * ws) * xs
+        if bias is not None:
+            want = want + bias.float()
+        assert torch.equal(_k().gemm_fp8_rows(x8, xs, w8, ws, bias), want.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("m,k,n", [s for s in SHAPES if s[1] % 128 == 0])
 def test_gemm_mx(m, k, n):
     g, x8, w8, b = _operands(m, k, n, m + k + n)
