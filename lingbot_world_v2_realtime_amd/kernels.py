@@ -28,7 +28,10 @@ _I32_ARRAYS = [ctypes_i32 * n for n in range(MAX_SEGMENTS + 1)]
 
 
 def _stream(t):
-    return _raw_stream(t.get_device())
+    idx = t.get_device()
+    if idx < 0:   # the raw call would take -1 as the current device
+        raise ValueError(f"expected a device tensor, got one on {t.device}")
+    return _raw_stream(idx)
 
 
 def _ptr(t):
@@ -392,6 +395,8 @@ def quant_mx_fp8(x, rows_pad=None, transposed=False):
 
 
 def _gemm_operands(x8, w8, bias):
+    if not x8.is_cuda:
+        raise ValueError("x8 must be a device tensor (the FP8 path has no CPU implementation)")
     if x8.dtype != torch.float8_e4m3fn or w8.dtype != torch.float8_e4m3fn:
         raise TypeError(f"x8 and w8 must be float8_e4m3fn, got {x8.dtype} / {w8.dtype}")
     if x8.dim() != 2 or w8.dim() != 2 or x8.shape[1] != w8.shape[1] or not x8.is_contiguous() \
