@@ -32,10 +32,18 @@ int lbw_gemm_fp8_mx(const uint8_t* x8, const uint8_t* x_scale_t, const uint8_t* 
 
 /*
  * lbw_quant_mx_fp8 with its scales written as [cols / 128][rows_pad][4] (cols a multiple of 128): the same bytes in
- * the order lbw_gemm_fp8_mx reads them. scale_t 4-byte aligned.
+ * the order lbw_gemm_fp8_mx reads them (which wants them 4-byte aligned).
  */
 int lbw_quant_mx_fp8_t(const void* x, int x_is_fp32, int64_t rows, int64_t rows_pad, int64_t cols, int64_t s_row,
                        uint8_t* x8, uint8_t* scale_t, void* stream);
+
+/*
+ * lbw_quant_mx_fp8_t, and in the same launch the scales of the other operand, w_scale_e8m0 [w_rows][cols / 32] as
+ * lbw_quant_mx_fp8 writes them, reordered into w_scale_t [cols / 128][w_rows][4]. Both 4-byte aligned.
+ */
+int lbw_quant_mx_fp8_tw(const void* x, int x_is_fp32, int64_t rows, int64_t rows_pad, int64_t cols, int64_t s_row,
+                        uint8_t* x8, uint8_t* scale_t, const uint8_t* w_scale_e8m0, int64_t w_rows, uint8_t* w_scale_t,
+                        void* stream);
 
 #ifdef __cplusplus
 }

@@ -42,6 +42,7 @@ GEMM_SIGNATURES = {
     "lbw_gemm_fp8_rows": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
     "lbw_gemm_fp8_mx": (_i32, [_p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
     "lbw_quant_mx_fp8_t": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _p]),
+    "lbw_quant_mx_fp8_tw": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _p, _p]),
 }
 
 

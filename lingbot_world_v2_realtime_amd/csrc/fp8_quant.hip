@@ -298,12 +298,24 @@ static void launch_quant_rows(const T* x, int64_t rows, int64_t cols, int64_t s_
 // infinite one). One thread per 32-value group; rows from `rows` up to `rows_pad` are written as zeros with scale
 // byte 127 (2^0), so a GEMM can take a row count padded to its tile. TRANS: the scales go out as [cols / 128][rows_pad]
 // dwords (a row's four scales of each 128 values together), the order in which lbw_gemm_fp8_mx loads them: 64 rows
-// are then 256 contiguous bytes instead of 64 cache lines (MX GEMM at 6032 x 8960 x 1536: 90.3 -> 76.8 us).
+// are then 256 contiguous bytes instead of 64 cache lines (MX GEMM at 6032 x 8960 x 1536: 90.3 -> 76.8 us). The
+// workgroups from q_blocks on put the scales of the other operand, ws [w_rows][cols / 128] dwords, into that order as
+// well: a linear's weight scales stay in one place, where a program may write them at any time, and take no launch of
+// their own on the way.
 template <typename T, bool TRANS>
 __global__ __launch_bounds__(256) void quant_mx_fp8_kernel(const T* __restrict__ x, int64_t rows, int64_t rows_pad,
                                                            int64_t cols, int64_t s_row, uint8_t* __restrict__ x8,
-                                                           uint8_t* __restrict__ e8) {
+                                                           uint8_t* __restrict__ e8, unsigned q_blocks,
+                                                           const uint32_t* __restrict__ ws, int64_t w_rows,
+                                                           uint32_t* __restrict__ wst) {
   const int64_t groups = cols / 32;
+  if constexpr (TRANS) {
+    if (blockIdx.x >= q_blocks) {   // in the order of the stores
+      const int64_t o = (int64_t)(blockIdx.x - q_blocks) * 256 + threadIdx.x, kb = o / w_rows;
+      if (kb < cols / 128) wst[o] = ws[(o - kb * w_rows) * (cols / 128) + kb];
+      return;
+    }
+  }
   const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (id >= rows_pad * groups) return;
   const int64_t row = id / groups, grp = id - row * groups;
@@ -385,22 +397,31 @@ extern "C" int lbw_quant_rows_fp8_gelu(const uint16_t* x, int64_t rows, int64_t 
   return LBW_OK;
 }
 
+// w_rows == 0: no weight scales to reorder.
 static int quant_mx(bool trans, const void* x, int x_is_fp32, int64_t rows, int64_t rows_pad, int64_t cols, int64_t s_row,
-                    uint8_t* x8, uint8_t* scale_e8m0, void* stream) {
-  if (!x || !x8 || !scale_e8m0) return LBW_E_NULL;
+                    uint8_t* x8, uint8_t* scale_e8m0, const uint8_t* w_scale, int64_t w_rows, uint8_t* w_scale_t,
+                    void* stream) {
+  if (!x || !x8 || !scale_e8m0 || (w_rows && (!w_scale || !w_scale_t))) return LBW_E_NULL;
   if (rows <= 0 || rows_pad < rows || cols <= 0 || cols % (trans ? 128 : 32) != 0 || s_row < cols) return LBW_E_SHAPE;
   if (rows_pad > ((int64_t)1 << 31) || rows_pad * (cols / 32) > ((int64_t)1 << 38)) return LBW_E_SHAPE;
-  if (s_row % 8 != 0 || ((uintptr_t)x & 15) || ((uintptr_t)x8 & 15)) return LBW_E_ALIGN;
+  if (w_rows < 0 || w_rows > ((int64_t)1 << 31) || w_rows * (cols / 32) > ((int64_t)1 << 38)) return LBW_E_SHAPE;
+  if (s_row % 8 != 0 || ((uintptr_t)x & 15) || ((uintptr_t)x8 & 15) || (((uintptr_t)w_scale | (uintptr_t)w_scale_t) & 3))
+    return LBW_E_ALIGN;
   if (const int dv = check_device()) return dv;
-  const int64_t n = rows_pad * (cols / 32);
-  const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+  const unsigned q_blocks = (unsigned)((rows_pad * (cols / 32) + 255) / 256);
+  const unsigned w_blocks = (unsigned)((w_rows * (cols / 128) + 255) / 256);
+  const dim3 grid(q_blocks + w_blocks), block(256);
   const hipStream_t st = (hipStream_t)stream;
+  const uint32_t* ws = (const uint32_t*)w_scale;
+  uint32_t* wst = (uint32_t*)w_scale_t;
   if (x_is_fp32) {
     const auto kern = trans ? quant_mx_fp8_kernel<float, true> : quant_mx_fp8_kernel<float, false>;
-    hipLaunchKernelGGL(kern, grid, block, 0, st, (const float*)x, rows, rows_pad, cols, s_row, x8, scale_e8m0);
+    hipLaunchKernelGGL(kern, grid, block, 0, st, (const float*)x, rows, rows_pad, cols, s_row, x8, scale_e8m0, q_blocks,
+                       ws, w_rows, wst);
   } else {
     const auto kern = trans ? quant_mx_fp8_kernel<uint16_t, true> : quant_mx_fp8_kernel<uint16_t, false>;
-    hipLaunchKernelGGL(kern, grid, block, 0, st, (const uint16_t*)x, rows, rows_pad, cols, s_row, x8, scale_e8m0);
+    hipLaunchKernelGGL(kern, grid, block, 0, st, (const uint16_t*)x, rows, rows_pad, cols, s_row, x8, scale_e8m0,
+                       q_blocks, ws, w_rows, wst);
   }
   if (hipGetLastError() != hipSuccess) return LBW_E_LAUNCH;
   return LBW_OK;
@@ -408,10 +429,17 @@ static int quant_mx(bool trans, const void* x, int x_is_fp32, int64_t rows, int6
 
 extern "C" int lbw_quant_mx_fp8(const void* x, int x_is_fp32, int64_t rows, int64_t rows_pad, int64_t cols,
                                 int64_t s_row, uint8_t* x8, uint8_t* scale_e8m0, void* stream) {
-  return quant_mx(false, x, x_is_fp32, rows, rows_pad, cols, s_row, x8, scale_e8m0, stream);
+  return quant_mx(false, x, x_is_fp32, rows, rows_pad, cols, s_row, x8, scale_e8m0, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int lbw_quant_mx_fp8_t(const void* x, int x_is_fp32, int64_t rows, int64_t rows_pad, int64_t cols,
                                   int64_t s_row, uint8_t* x8, uint8_t* scale_t, void* stream) {
-  return quant_mx(true, x, x_is_fp32, rows, rows_pad, cols, s_row, x8, scale_t, stream);
+  return quant_mx(true, x, x_is_fp32, rows, rows_pad, cols, s_row, x8, scale_t, nullptr, 0, nullptr, stream);
+}
+
+extern "C" int lbw_quant_mx_fp8_tw(const void* x, int x_is_fp32, int64_t rows, int64_t rows_pad, int64_t cols,
+                                   int64_t s_row, uint8_t* x8, uint8_t* scale_t, const uint8_t* w_scale_e8m0,
+                                   int64_t w_rows, uint8_t* w_scale_t, void* stream) {
+  if (w_rows <= 0) return LBW_E_SHAPE;
+  return quant_mx(true, x, x_is_fp32, rows, rows_pad, cols, s_row, x8, scale_t, w_scale_e8m0, w_rows, w_scale_t, stream);
 }

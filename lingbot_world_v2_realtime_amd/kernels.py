@@ -366,11 +366,13 @@ def quant_rows_fp8_gelu(x):
     return x8, scale
 
 
-def quant_mx_fp8(x, rows_pad=None, transposed=False):
+def quant_mx_fp8(x, rows_pad=None, transposed=False, w_scale=None):
     """MXFP8 of a 2-d bf16 / fp32 device tensor x [rows, cols] (cols a multiple of 32, unit column stride):
     (x8 float8_e4m3fn [rows_pad, cols], scale float8_e8m0fnu [rows_pad, cols / 32]), one power-of-two scale per 32
     values; rows past `rows` (up to rows_pad, default rows) are zero with scale 1. transposed (cols a multiple of
-    128): the scale bytes as uint8 [cols / 128, rows_pad, 4], the order gemm_fp8_mx takes."""
+    128): the scale bytes as uint8 [cols / 128, rows_pad, 4], the order gemm_fp8_mx takes; with w_scale (another
+    operand's scales [N, cols / 32], float8_e8m0fnu) also those in that order, uint8 [cols / 128, N, 4], from the same
+    launch: (x8, scale, w_scale_t)."""
     lib = _lib.load()
     if not x.is_cuda:
         raise ValueError("x must be a device tensor (the FP8 path has no CPU implementation)")
@@ -383,10 +385,22 @@ def quant_mx_fp8(x, rows_pad=None, transposed=False):
     x8 = torch.empty(rows_pad, cols, dtype=torch.float8_e4m3fn, device=x.device)
     if transposed:
         e8 = torch.empty(cols // 128, rows_pad, 4, dtype=torch.uint8, device=x.device)
-        st = lib.lbw_quant_mx_fp8_t(_ptr(x), int(x.dtype == torch.float32), rows, rows_pad, cols, x.stride(0),
-                                    _ptr(x8), _ptr(e8), _stream(x))
-        _lib.check(st, "lbw_quant_mx_fp8_t")
-        return x8, e8
+        if w_scale is None:
+            st = lib.lbw_quant_mx_fp8_t(_ptr(x), int(x.dtype == torch.float32), rows, rows_pad, cols, x.stride(0),
+                                        _ptr(x8), _ptr(e8), _stream(x))
+            _lib.check(st, "lbw_quant_mx_fp8_t")
+            return x8, e8
+        if w_scale.dtype != torch.float8_e8m0fnu or w_scale.dim() != 2 or w_scale.shape[1] * 32 != cols:
+            raise ValueError(f"w_scale must be float8_e8m0fnu [N, {cols // 32}], got {w_scale.dtype} "
+                             f"{tuple(w_scale.shape)}")
+        _same_device("quant_mx_fp8", x, w_scale)
+        if not w_scale.is_contiguous() or w_scale.data_ptr() % 4:   # the kernel loads dwords
+            w_scale = w_scale.clone(memory_format=torch.contiguous_format)
+        wt = torch.empty(cols // 128, w_scale.shape[0], 4, dtype=torch.uint8, device=x.device)
+        st = lib.lbw_quant_mx_fp8_tw(_ptr(x), int(x.dtype == torch.float32), rows, rows_pad, cols, x.stride(0),
+                                     _ptr(x8), _ptr(e8), _ptr(w_scale), w_scale.shape[0], _ptr(wt), _stream(x))
+        _lib.check(st, "lbw_quant_mx_fp8_tw")
+        return x8, e8, wt
     e8 = torch.empty(rows_pad, cols // 32, dtype=torch.uint8, device=x.device)
     st = lib.lbw_quant_mx_fp8(_ptr(x), int(x.dtype == torch.float32), rows, rows_pad, cols, x.stride(0), _ptr(x8),
                               _ptr(e8), _stream(x))

@@ -110,8 +110,8 @@ def _pad(n, m):
 class MXFP8Linear(torch.nn.Module):
     """MXFP8 replacement of an nn.Linear (lingbot/layers/linear.py:53-73): e4m3 with one power-of-two (E8M0)
     scale per 32 values along K for the weights (once) and the activations (every call). The quantisation is
-    lbw_quant_mx_fp8 (the activations' scales in the GEMM's order: lbw_quant_mx_fp8_t), the GEMM lbw_gemm_fp8_mx with
-    the bias in its epilogue; a bias that records a gradient is added after it instead.
+    lbw_quant_mx_fp8 (in a call lbw_quant_mx_fp8_tw: both operands' scales in the GEMM's order), the GEMM
+    lbw_gemm_fp8_mx with the bias in its epilogue; a bias that records a gradient is added after it instead.
     A K that is not a multiple of 128 (the GEMM's scale tile) is padded with zero columns, weights once and
     activations per call: a zero group quantises to zeros, so the product is unchanged."""
 
@@ -127,19 +127,8 @@ class MXFP8Linear(torch.nn.Module):
         w8, ws = kernels.quant_mx_fp8(w.contiguous(), _pad(n, MX_ROWS))
         self.register_buffer("w8", w8)             # [Np, Kp]
         self.register_buffer("w_scale", ws)        # [Np, Kp / 32] e8m0
-        self.register_buffer("w_scale_t", None, persistent=False)   # the same bytes as the GEMM reads them
-        self._order_scales()
         self.bias = lin.bias
         self.in_features, self.out_features = lin.in_features, lin.out_features
-
-    def _order_scales(self):
-        """w_scale's bytes as [Kp / 128, Np, 4], made again whenever weights are loaded."""
-        n = self.w_scale.shape[0]
-        self.w_scale_t = self.w_scale.view(torch.uint8).view(n, -1, 4).transpose(0, 1).contiguous()
-
-    def _load_from_state_dict(self, *args, **kwargs):
-        super()._load_from_state_dict(*args, **kwargs)
-        self._order_scales()
 
     def forward(self, x):
         shape = x.shape
@@ -148,10 +137,11 @@ class MXFP8Linear(torch.nn.Module):
             x2 = x2.float()
         if self.k_pad:
             x2 = torch.nn.functional.pad(x2, (0, self.k_pad))
-        x8, xs = kernels.quant_mx_fp8(x2.contiguous(), transposed=True)
+        # the weights' scales go into the GEMM's order on every call: a kept copy would not follow writes to w_scale
+        x8, xs, ws = kernels.quant_mx_fp8(x2.contiguous(), transposed=True, w_scale=self.w_scale)
         bias = None if self.bias is None else self.bias.to(torch.bfloat16)
         fused = bias is not None and not _records_grad(bias) and self.out_features == self.w8.shape[0]
-        y = kernels.gemm_fp8_mx(x8, xs, self.w8, self.w_scale_t, bias if fused else None)
+        y = kernels.gemm_fp8_mx(x8, xs, self.w8, ws, bias if fused else None)
         y = y[:, :self.out_features]
         if bias is not None and not fused:
             y = y + bias

@@ -104,6 +104,47 @@ def test_quant_mx_transposed_scales():
         assert torch.equal(ae.view(torch.uint8).view(128, -1, 4).transpose(0, 1), be)
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 128, 1), (77, 1152, 384), (300, 1536, 8960), (6032, 128, 257)])
+def test_quant_mx_other_operands_scales(m, k, n):
+    """The other operand's scales reordered in the quantiser's launch, also from a strided and a misaligned view."""
+    x = torch.randn(m, k, device=DEV).to(torch.bfloat16)
+    e = torch.randint(0, 256, (n, k // 32), device=DEV, dtype=torch.uint8)
+    wide, odd = torch.zeros(n, k // 16, device=DEV, dtype=torch.uint8), torch.zeros(n * (k // 32) + 1, device=DEV,
+                                                                                   dtype=torch.uint8)
+    wide[:, :k // 32], odd[1:] = e, e.view(-1)
+    want = e.view(n, -1, 4).transpose(0, 1)
+    a8, ae = _k().quant_mx_fp8(x, transposed=True)
+    for w in (e, wide[:, :k // 32], odd[1:].view(n, -1)):
+        b8, be, wt = _k().quant_mx_fp8(x, transposed=True, w_scale=w.view(torch.float8_e8m0fnu))
+        assert torch.equal(a8.view(torch.uint8), b8.view(torch.uint8)) and torch.equal(ae, be) and torch.equal(wt, want)
+
+
+def test_mx_scales_follow_writes():
+    """MXFP8Linear multiplies by what w8 and w_scale hold at the call: after in-place writes through state_dict(), and
+    after writes that no version counter sees (.data, as a collective's), as a module built from those weights; also with
+    the buffers exchanged, and in a copy."""
+    import copy
+    from lingbot_world_v2_realtime_amd.layers.linear import MXFP8Linear
+    with torch.no_grad():
+        a, b = (torch.nn.Linear(1536, 1000, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        b.weight.mul_(torch.exp2(torch.randint(-6, 7, (1000, 1), device=DEV).to(torch.bfloat16)))
+        b.bias.copy_(a.bias)
+        src = MXFP8Linear(b)
+        x = torch.randn(65, 1536, device=DEV).to(torch.bfloat16)
+        want = src(x)
+        for write in ("state_dict", "data", "exchange"):
+            mx = MXFP8Linear(a)
+            assert not torch.equal(mx(x), want)
+            for name in ("w8", "w_scale"):
+                if write == "exchange":
+                    setattr(mx, name, getattr(src, name).clone())
+                else:
+                    dst = mx.state_dict()[name] if write == "state_dict" else getattr(mx, name).data
+                    dst.view(torch.uint8).copy_(getattr(src, name).view(torch.uint8))
+            assert torch.equal(mx(x), want), write
+        assert torch.equal(copy.deepcopy(mx)(x), want)
+
+
 def test_nonfinite_rows_stay_in_their_row():
     """A row whose scale is inf or NaN gives a NaN row and leaves the others as they are."""
     g, x8, w8, b = _operands(300, 1536, 1536, 5)
