@@ -4,14 +4,18 @@ scale per 32 values along K for both; the GEMM accumulates in fp32 and writes bf
 
 On MI355X the per-row quantisation of weights and activations is a HIP kernel (lbw_quant_rows_fp8, bit for bit the
 reference's formula) and the GEMM another (lbw_gemm_fp8_rows / lbw_gemm_fp8_mx), with the scales and the bias in its
-epilogue. Only a rowwise call that records a gradient for the bias still runs hipBLASLt's
-rowwise-scaled FP8 GEMM through torch._scaled_mm, which autograd knows (and refuses to differentiate); for that call,
-and for a program's own _scaled_mm calls, use_tuned_gemms() picks the hipBLASLt solutions of fp8_gemm_solutions.csv
-(tune_gemms() writes such a table).
+epilogue. hipBLASLt's FP8 GEMM, through torch._scaled_mm, still runs where the kernel may not take a tensor by its
+address or does not take its layout: a rowwise call whose bias records a gradient or carries a forward-mode tangent
+(which torch refuses to differentiate), weights, scales or bias inside a torch.func transform or of a tensor subclass,
+weights that are not contiguous, a rowwise out_features that is not a multiple of 16 or a bias of other than one
+dimension. The MX form adds such a bias to the kernel's product instead. For those calls, and for a program's own
+_scaled_mm calls, use_tuned_gemms() picks the hipBLASLt solutions of fp8_gemm_solutions.csv (tune_gemms() writes such a
+table).
 """
 import os
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import kernels
 
@@ -86,17 +90,33 @@ class FP8Linear(torch.nn.Module):
             if x2.dtype not in (torch.bfloat16, torch.float32):
                 x2 = x2.float()
             x8, x_scale = kernels.quant_rows_fp8(x2.contiguous())
-        bias = None if self.bias is None else self.bias.to(torch.bfloat16)
-        if _records_grad(bias) or not self.w8.is_contiguous() or self.out_features % 16:
-            y = torch._scaled_mm(x8, self.w8.t(), scale_a=x_scale, scale_b=self.w_scale_t, bias=bias,
-                                 out_dtype=torch.bfloat16)
+        w8, w_scale, bias = self.w8, self.w_scale_t, self.bias   # (a module's attributes cost ~0.5 us a look)
+        if bias is not None:
+            bias = bias.to(torch.bfloat16)
+        if _plain(bias, w8, w_scale) and w8.is_contiguous() and self.out_features % 16 == 0 and \
+                (bias is None or bias.dim() == 1):
+            y = kernels.gemm_fp8_rows(x8, x_scale, w8, w_scale, bias)
         else:
-            y = kernels.gemm_fp8_rows(x8, x_scale, self.w8, self.w_scale_t, bias)
-        return y if len(shape) == 2 else y.view(*shape[:-1], y.shape[1])
+            y = torch._scaled_mm(x8, w8.t(), scale_a=x_scale, scale_b=w_scale, bias=bias, out_dtype=torch.bfloat16)
+        return y if len(shape) == 2 else y.reshape(*shape[:-1], y.shape[1])
 
 
-def _records_grad(bias):
-    return bias is not None and bias.requires_grad and torch.is_grad_enabled()
+_func_level = torch._C._functorch.peek_interpreter_stack
+
+
+def _plain(*tensors):
+    """Whether a kernel may take these (None: absent) by their address: none records a gradient, carries a forward-mode
+    tangent, stands for others inside a torch.func transform, or is of a tensor subclass. Others stay with torch's own
+    operations, which know what to do with them or refuse."""
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in (torch.Tensor, torch.nn.Parameter) or (grad and t.requires_grad)):
+            return False
+    # the rest only exists inside a transform or a dual level: two cheap looks instead of two calls a tensor (~1.4 us)
+    if _func_level() is None and forward_ad._current_level < 0:
+        return True
+    return not any(torch._C._functorch.is_functorch_wrapped_tensor(t) or
+                   forward_ad.unpack_dual(t).tangent is not None for t in tensors if t is not None)
 
 
 MX_ROWS = 128   # weight rows are padded to this (the library MX GEMM's row tile, which the stored weights keep)
@@ -111,7 +131,7 @@ class MXFP8Linear(torch.nn.Module):
     """MXFP8 replacement of an nn.Linear (lingbot/layers/linear.py:53-73): e4m3 with one power-of-two (E8M0)
     scale per 32 values along K for the weights (once) and the activations (every call). The quantisation is
     lbw_quant_mx_fp8 (in a call lbw_quant_mx_fp8_tw: both operands' scales in the GEMM's order), the GEMM
-    lbw_gemm_fp8_mx with the bias in its epilogue; a bias that records a gradient is added after it instead.
+    lbw_gemm_fp8_mx with the bias in its epilogue; a bias that is not a plain [out_features] tensor (_plain) is added after it.
     A K that is not a multiple of 128 (the GEMM's scale tile) is padded with zero columns, weights once and
     activations per call: a zero group quantises to zeros, so the product is unchanged."""
 
@@ -137,13 +157,23 @@ class MXFP8Linear(torch.nn.Module):
             x2 = x2.float()
         if self.k_pad:
             x2 = torch.nn.functional.pad(x2, (0, self.k_pad))
+        w8, w_scale, bias = self.w8, self.w_scale, self.bias
+        if bias is not None:
+            bias = bias.to(torch.bfloat16)
+        if not _plain(w8, w_scale) or not w8.is_contiguous():
+            m = x2.shape[0]
+            x8, xs = kernels.quant_mx_fp8(x2.contiguous(), _pad(m, MX_ROWS))
+            y = torch._scaled_mm(x8, w8.t(), scale_a=xs, scale_b=w_scale, out_dtype=torch.bfloat16)[:m]
+            return self._add_bias(y, bias, shape)
         # the weights' scales go into the GEMM's order on every call: a kept copy would not follow writes to w_scale
-        x8, xs, ws = kernels.quant_mx_fp8(x2.contiguous(), transposed=True, w_scale=self.w_scale)
-        bias = None if self.bias is None else self.bias.to(torch.bfloat16)
-        fused = bias is not None and not _records_grad(bias) and self.out_features == self.w8.shape[0]
-        y = kernels.gemm_fp8_mx(x8, xs, self.w8, ws, bias if fused else None)
+        x8, xs, ws = kernels.quant_mx_fp8(x2.contiguous(), transposed=True, w_scale=w_scale)
+        fused = bias is not None and _plain(bias) and bias.shape == w8.shape[:1] == (self.out_features,)
+        y = kernels.gemm_fp8_mx(x8, xs, w8, ws, bias if fused else None)
+        return self._add_bias(y, None if fused else bias, shape)
+
+    def _add_bias(self, y, bias, shape):
         y = y[:, :self.out_features]
-        if bias is not None and not fused:
+        if bias is not None:
             y = y + bias
         return y.reshape(*shape[:-1], self.out_features)
 

@@ -181,3 +181,31 @@ def test_linears_run_the_kernel(m, k, n):
     assert grad.requires_grad
     assert (grad.float() - y.float()).abs().max() <= 2.0 ** -7 * y.float().abs().max()
     assert mx(x).requires_grad
+
+
+def test_bias_with_a_tangent_or_under_vmap():
+    """What the kernel may not take by its address: MXFP8Linear adds it to the product, FP8Linear leaves it to
+    torch._scaled_mm, which refuses the derivative."""
+    from torch.autograd import forward_ad
+    from lingbot_world_v2_realtime_amd.layers.linear import FP8Linear, MXFP8Linear
+    lin = torch.nn.Linear(1536, 1024, device=DEV, dtype=torch.bfloat16).requires_grad_(False)
+    x = torch.randn(130, 1536, device=DEV).to(torch.bfloat16)
+    mx, f, b = MXFP8Linear(lin), FP8Linear(lin), lin.bias.detach().clone()
+    t, want, rows = torch.randn_like(b), mx(x), f(x)
+    del mx.bias, f.bias
+    with forward_ad.dual_level():
+        mx.bias = f.bias = forward_ad.make_dual(b, t)
+        out = forward_ad.unpack_dual(mx(x))
+        assert torch.equal(out.primal, want) and torch.equal(out.tangent, t.expand(130, -1))
+        with pytest.raises(NotImplementedError):
+            f(x)
+
+    def call(module):
+        def fn(bias):
+            module.bias = bias
+            return module(x)
+        return fn
+
+    two = torch.vmap(call(mx))(torch.stack([b, b + 1]))
+    assert torch.equal(two[0], want) and torch.equal(two[1], call(mx)(b + 1))
+    assert torch.equal(call(f)(b.view(1, -1)), rows)   # a bias of n values in two dimensions: torch's product
