@@ -1,6 +1,7 @@
 """Thin torch-side wrappers over the C-ABI: device memory and the current stream come from torch, the work is
 done by the HIP kernels in liblbw_attn.so. Nothing here computes on the CPU."""
 import ctypes
+import operator
 
 import torch
 
@@ -124,9 +125,11 @@ class RingCache:
 
     def layer_ptrs(self, layer):
         """Device addresses of one layer's (k8, k_scale, km, v8, v8lo or None, v_scale)."""
-        if not -self.layers <= layer < self.layers:
+        i = operator.index(layer)   # a numpy integer or a 0-d tensor, as an index would take, must not reach the address
+        if not -self.layers <= i < self.layers:
             raise IndexError(f"layer {layer} is out of range for {self.layers} layers")
-        i = layer + self.layers if layer < 0 else layer
+        if i < 0:
+            i += self.layers
         lo = self.v8lo
         return (self.k8.data_ptr() + i * self.k8.stride(0), self.k_scale.data_ptr() + 4 * i * self.k_scale.stride(0),
                 self.km.data_ptr() + 4 * i * self.km.stride(0), self.v8.data_ptr() + i * self.v8.stride(0),

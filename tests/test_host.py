@@ -24,6 +24,22 @@ def test_ring_layout_sizes():
         kernels.RingCache(1, 1, 1, 64, 2, "cpu", v_terms=3)
 
 
+def test_ring_layer_addresses():
+    """layer_ptrs gives the addresses of layer_view's tensors, for every kind of integer an index may be."""
+    import numpy as np
+    for terms in (1, 2):
+        r = kernels.RingCache(layers=3, batch=2, heads=5, cap=192, slots=4, device="cpu", v_terms=terms)
+        for layer in (0, 2, -1, -3, np.int64(1), np.int32(2), torch.tensor(1), torch.tensor(-2)):
+            got = r.layer_ptrs(layer)
+            assert got == tuple(None if t is None else t.data_ptr() for t in r.layer_view(layer)), layer
+            assert all(p is None or type(p) is int for p in got)
+        for bad in (3, -4, np.int64(3)):
+            with pytest.raises(IndexError):
+                r.layer_ptrs(bad)
+        with pytest.raises((IndexError, TypeError)):
+            r.layer_ptrs(1.0)
+
+
 def test_ring_slot_rotation():
     """Saved chunks oldest first, then the current one; with 4 slots the 4th commit evicts the oldest."""
     ring = kv_quant.QuantKVRing(num_layers=1, batch=1, heads=1, chunk_len=100, slots=4, device="cpu")
