@@ -412,6 +412,8 @@ def quant_mx_fp8(x, rows_pad=None, transposed=False, w_scale=None):
 
 
 def _gemm_operands(x8, w8, bias):
+    """The GEMM's operands, checked; weights and a bias at an address the kernel does not load from (views of a larger
+    buffer, say a flat checkpoint) as copies."""
     if not x8.is_cuda:
         raise ValueError("x8 must be a device tensor (the FP8 path has no CPU implementation)")
     if x8.dtype != torch.float8_e4m3fn or w8.dtype != torch.float8_e4m3fn:
@@ -424,14 +426,14 @@ def _gemm_operands(x8, w8, bias):
             raise ValueError(f"bias must be bfloat16 ({w8.shape[0]},), got {bias.dtype} {tuple(bias.shape)}")
         if not bias.is_contiguous() or bias.data_ptr() % 4:   # the kernel loads pairs
             bias = bias.clone(memory_format=torch.contiguous_format)
-    return bias
+    return w8.clone() if w8.data_ptr() % 16 else w8, bias
 
 
 def gemm_fp8_rows(x8, x_scale, w8, w_scale, bias=None):
     """The rowwise-scaled FP8 product (lbw_gemm_fp8_rows): x8 [M, K] and w8 [N, K] float8_e4m3fn, x_scale M and w_scale
     N fp32 values, bias bf16 [N] or None -> bf16 [M, N] = (x8 w8^T w_scale) x_scale + bias: fp32, in this order."""
     m, n = x8.shape[0], w8.shape[0]
-    bias = _gemm_operands(x8, w8, bias)
+    w8, bias = _gemm_operands(x8, w8, bias)
     if x_scale.dtype != torch.float32 or w_scale.dtype != torch.float32 or x_scale.numel() != m \
             or w_scale.numel() != n or not x_scale.is_contiguous() or not w_scale.is_contiguous():
         raise ValueError(f"scales must be {m} and {n} contiguous fp32 values")
@@ -447,7 +449,7 @@ def gemm_fp8_mx(x8, x_scale_t, w8, w_scale_t, bias=None):
     """The MX-scaled FP8 product (lbw_gemm_fp8_mx): x8 [M, K] and w8 [N, K] float8_e4m3fn, their E8M0 scale bytes uint8
     [K / 128, M, 4] and [K / 128, N, 4] (quant_mx_fp8(transposed=True)), bias bf16 [N] or None -> bf16 [M, N]."""
     m, n, k = x8.shape[0], w8.shape[0], x8.shape[1]
-    bias = _gemm_operands(x8, w8, bias)
+    w8, bias = _gemm_operands(x8, w8, bias)
     for s, rows in ((x_scale_t, m), (w_scale_t, n)):
         if s.dtype != torch.uint8 or tuple(s.shape) != (k // 128, rows, 4) or not s.is_contiguous():
             raise ValueError(f"scales must be contiguous uint8 {(k // 128, rows, 4)}, got {s.dtype} {tuple(s.shape)}")

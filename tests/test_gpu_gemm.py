@@ -209,3 +209,16 @@ def test_bias_with_a_tangent_or_under_vmap():
     two = torch.vmap(call(mx))(torch.stack([b, b + 1]))
     assert torch.equal(two[0], want) and torch.equal(two[1], call(mx)(b + 1))
     assert torch.equal(call(f)(b.view(1, -1)), rows)   # a bias of n values in two dimensions: torch's product
+
+
+def test_weights_at_any_address():
+    """Weights that are a view into a larger buffer, at an address that is not a multiple of 16."""
+    from lingbot_world_v2_realtime_amd.layers.linear import FP8Linear, MXFP8Linear
+    lin = torch.nn.Linear(1536, 1024, device=DEV, dtype=torch.bfloat16).requires_grad_(False)
+    x = torch.randn(65, 1536, device=DEV).to(torch.bfloat16)
+    for module in (FP8Linear(lin), MXFP8Linear(lin)):
+        want = module(x)
+        flat = torch.zeros(module.w8.numel() + 1, dtype=torch.uint8, device=DEV)
+        flat[1:] = module.w8.view(torch.uint8).view(-1)
+        module.w8 = flat[1:].view(torch.float8_e4m3fn).view(module.w8.shape)
+        assert module.w8.data_ptr() % 16 and torch.equal(module(x), want)
