@@ -12,14 +12,15 @@ import pytest
 from lingbot_world_v2_realtime_amd import _lib
 
 HEADER = os.path.join(os.path.dirname(__file__), "..", "include", "lbw_attn.h")
+GEMM_HEADER = os.path.join(os.path.dirname(__file__), "..", "include", "lbw_gemm.h")
 
 OK, E_NULL, E_SHAPE, E_ALIGN, E_DEVICE, E_LAUNCH, E_SEGMENTS, E_SCRATCH = range(8)
 FAKE = 1 << 20          # a 16-byte aligned non-null address; never dereferenced on the paths tested here
 
 
-def declared_functions():
+def declared_functions(header=HEADER):
     """{name: number of parameters} of every function prototype in the header."""
-    src = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    src = re.sub(r"/\*.*?\*/", "", open(header).read(), flags=re.S)
     out = {}
     for m in re.finditer(r"^\s*(?:const\s+)?\w+\s*\*?\s*(lbw_\w+)\s*\(([^)]*)\)\s*;", src, flags=re.M):
         params = m.group(2).strip()
@@ -44,6 +45,13 @@ def test_header_declarations_are_bound_and_exported(lib):
     nm = subprocess.run(["nm", "-D", "--defined-only", _lib.LIB_PATH], capture_output=True, text=True).stdout
     exported = {line.split()[-1] for line in nm.splitlines() if " T " in line and "lbw_" in line}
     assert set(decl) <= exported
+
+
+def test_gemm_header_declarations_are_bound_and_exported(lib):
+    decl = declared_functions(GEMM_HEADER)
+    assert len(decl) == 4 and set(decl) == set(_lib.GEMM_SIGNATURES)
+    for name, n in decl.items():
+        assert len(_lib.GEMM_SIGNATURES[name][1]) == n and hasattr(lib, name), name
 
 
 def test_status_strings_and_version(lib):
@@ -216,6 +224,66 @@ def test_quant_rows_fp8_argument_checks(lib):
     assert mx(x8=FAKE + 8) == E_ALIGN
     if hip_device_count() == 0:
         assert mx() == E_DEVICE
+
+
+def gemm(lib, name, **kw):
+    a = dict(x8=FAKE, xs=FAKE, w8=FAKE, ws=FAKE, bias=FAKE, m=100, n=256, k=384, out=FAKE)
+    a.update(kw)
+    return getattr(lib, name)(a["x8"], a["xs"], a["w8"], a["ws"], a["bias"], a["m"], a["n"], a["k"], a["out"], None)
+
+
+@pytest.mark.parametrize("name", ["lbw_gemm_fp8_rows", "lbw_gemm_fp8_mx"])
+def test_gemm_argument_checks(lib, name):
+    for p in ("x8", "xs", "w8", "ws", "out"):
+        assert gemm(lib, name, **{p: None}) == E_NULL
+    for p in ("m", "n", "k"):
+        assert gemm(lib, name, **{p: 0}) == E_SHAPE
+        assert gemm(lib, name, **{p: -16}) == E_SHAPE
+    assert gemm(lib, name, n=264) == E_SHAPE               # multiples of 16
+    assert gemm(lib, name, k=392) == E_SHAPE
+    assert gemm(lib, name, n=(1 << 22) + 16) == E_SHAPE
+    assert gemm(lib, name, k=(1 << 22) + 128) == E_SHAPE
+    assert gemm(lib, name, m=(1 << 30) + 1) == E_SHAPE
+    assert gemm(lib, name, m=1 << 30, n=1 << 22) == E_SHAPE   # the tile count
+    for p in ("x8", "w8", "out"):
+        assert gemm(lib, name, **{p: FAKE + 8}) == E_ALIGN
+    for p in ("xs", "ws", "bias"):
+        assert gemm(lib, name, **{p: FAKE + 2}) == E_ALIGN
+    if name == "lbw_gemm_fp8_mx":
+        assert gemm(lib, name, k=192) in (E_SHAPE, E_DEVICE)   # whole 128-value scale tiles (checked after the device)
+    if hip_device_count() == 0:
+        assert gemm(lib, name) == E_DEVICE
+        assert gemm(lib, name, bias=None) == E_DEVICE
+
+
+def test_quant_mx_transposed_argument_checks(lib):
+    def mx(weights, **kw):
+        a = dict(x=FAKE, rows=10, pad=128, cols=256, s=256, x8=FAKE, sc=FAKE, ws=FAKE, wn=64, wt=FAKE)
+        a.update(kw)
+        args = (a["x"], 0, a["rows"], a["pad"], a["cols"], a["s"], a["x8"], a["sc"])
+        if weights:
+            return lib.lbw_quant_mx_fp8_tw(*args, a["ws"], a["wn"], a["wt"], None)
+        return lib.lbw_quant_mx_fp8_t(*args, None)
+
+    for weights in (False, True):
+        for p in ("x", "x8", "sc"):
+            assert mx(weights, **{p: None}) == E_NULL
+        assert mx(weights, cols=160, s=160) == E_SHAPE         # whole 128-value scale tiles
+        assert mx(weights, rows=0) == E_SHAPE
+        assert mx(weights, pad=5) == E_SHAPE
+        assert mx(weights, s=200) == E_SHAPE
+        assert mx(weights, s=260) == E_ALIGN
+        assert mx(weights, x=FAKE + 8) == E_ALIGN
+        assert mx(weights, x8=FAKE + 8) == E_ALIGN
+        if hip_device_count() == 0:
+            assert mx(weights) == E_DEVICE
+    assert mx(True, ws=None) == E_NULL
+    assert mx(True, wt=None) == E_NULL
+    assert mx(True, wn=0) == E_SHAPE
+    assert mx(True, wn=-1) == E_SHAPE
+    assert mx(True, wn=(1 << 31) + 1) == E_SHAPE
+    assert mx(True, ws=FAKE + 2) == E_ALIGN
+    assert mx(True, wt=FAKE + 2) == E_ALIGN
 
 
 def attn(lib, logits=None, **kw):

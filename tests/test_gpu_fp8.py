@@ -1,6 +1,6 @@
 """The FP8 linear path on the device: the rowwise e4m3 quantisation kernel (lbw_quant_rows_fp8, through the
-C-ABI) bit for bit against the oracle, and FP8Linear (that kernel + hipBLASLt's rowwise-scaled FP8 GEMM) against
-the fp32 product of the same quantised operands."""
+C-ABI) bit for bit against the oracle, and FP8Linear and MXFP8Linear against the fp32 product of the same quantised
+operands, without gradients (the FP8 GEMM kernels) and with a bias that records one (rowwise: torch._scaled_mm)."""
 import pytest
 import torch
 
@@ -59,8 +59,10 @@ def test_quant_rows_strided_view():
     assert torch.equal(x8.view(torch.uint8).cpu(), rb) and torch.equal(sc.cpu(), rs)
 
 
-@pytest.mark.parametrize("m,k,n,bias", [(6032, 1536, 1536, True), (333, 1536, 8960, False), (64, 8960, 1536, True)])
-def test_fp8_linear(m, k, n, bias):
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("m,k,n,bias", [(6032, 1536, 1536, True), (333, 1536, 8960, False), (64, 8960, 1536, True),
+                                        (6032, 1536, 8960, True), (6032, 8960, 1536, True)])
+def test_fp8_linear(m, k, n, bias, grad):
     from lingbot_world_v2_realtime_amd.layers.linear import FP8Linear
     g = torch.Generator().manual_seed(m)
     lin = torch.nn.Linear(k, n, bias=bias).to(torch.bfloat16)
@@ -73,7 +75,8 @@ def test_fp8_linear(m, k, n, bias):
     # a 3-d activation [2, m / 2, k] when m is even (the DiT's [B, L, C]), else 2-d
     shape = (2, m // 2, k) if m % 2 == 0 else (m, k)
     x = torch.randn(*shape, generator=g).to(torch.bfloat16)
-    y = f(x.to(DEV))
+    with torch.set_grad_enabled(grad):
+        y = f(x.to(DEV)).detach()
     torch.cuda.synchronize()
     assert y.dtype == torch.bfloat16 and y.shape == (*x.shape[:-1], n)
     # the same quantised operands in fp32 on the CPU
@@ -90,8 +93,8 @@ def test_fp8_linear(m, k, n, bias):
     if bias:
         full = full + lin.bias.detach().cpu().float()
     rel = ((y.reshape(-1, n).float().cpu() - full).norm() / full.norm()).item()
-    record(f"FP8Linear {m}x{k}x{n}: vs same-operand fp32 max {e.max().item():.2e} (|ref| max {scale:.2e}); "
-           f"vs bf16 linear rel-L2 {rel:.2e}")
+    record(f"FP8Linear {m}x{k}x{n} {'grad' if grad else 'no_grad'}: vs same-operand fp32 max {e.max().item():.2e} "
+           f"(|ref| max {scale:.2e}); vs bf16 linear rel-L2 {rel:.2e}")
     assert rel < 6e-2
 
 
@@ -153,8 +156,9 @@ def test_quant_mx_bit_exact(rows, rows_pad, cols, dtype):
     assert not x8.view(torch.uint8)[rows:].any() and (e8.view(torch.uint8)[rows:] == 127).all()
 
 
-@pytest.mark.parametrize("m,k,n,bias", [(6032, 1536, 1536, True), (100, 1536, 8960, False)])
-def test_mxfp8_linear(m, k, n, bias):
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("m,k,n,bias", [(6032, 1536, 1536, True), (100, 1536, 8960, False), (1508, 1536, 8960, True)])
+def test_mxfp8_linear(m, k, n, bias, grad):
     from lingbot_world_v2_realtime_amd.layers.linear import MXFP8Linear
     g = torch.Generator().manual_seed(m + 1)
     lin = torch.nn.Linear(k, n, bias=bias).to(torch.bfloat16)
@@ -164,7 +168,8 @@ def test_mxfp8_linear(m, k, n, bias):
             lin.bias.copy_(torch.randn(n, generator=g) * 0.1)
     f = MXFP8Linear(lin.to(DEV))
     x = torch.randn(m, k, generator=g).to(torch.bfloat16)
-    y = f(x.to(DEV))
+    with torch.set_grad_enabled(grad):
+        y = f(x.to(DEV)).detach()
     torch.cuda.synchronize()
     assert y.shape == (m, n) and y.dtype == torch.bfloat16
     xb, xe = fp8.quant_mx(x)
@@ -173,7 +178,8 @@ def test_mxfp8_linear(m, k, n, bias):
     if bias:
         ref = ref + lin.bias.detach().cpu().float()
     e = (y.float().cpu() - ref).abs()
-    record(f"MXFP8Linear {m}x{k}x{n}: vs same-operand fp32 max {e.max().item():.2e} (|ref| max {ref.abs().max().item():.2e})")
+    record(f"MXFP8Linear {m}x{k}x{n} {'grad' if grad else 'no_grad'}: vs same-operand fp32 max {e.max().item():.2e} "
+           f"(|ref| max {ref.abs().max().item():.2e})")
     assert e.max().item() <= 1e-2 * ref.abs().max().item()
 
 

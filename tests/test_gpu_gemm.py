@@ -39,9 +39,9 @@ def _check(y, x, w, bias, align=2.0 ** -15, rnd=2.0 ** -8):
     assert bool(((y.double() - ref).abs() <= tol).all()), float(((y.double() - ref).abs() - tol).max())
 
 
-# one K share / two (K >= 4096) at 64 x 64; 128 x 128; 192 x 192 in one and more rounds; 256 x 256, full and ragged, with a
+# one K share / two (K >= 4096; 4224: an odd number of stages, the second share's last one past K) at 64 x 64; 128 x 128; 192 x 192 in one and more rounds; 256 x 256, full and ragged, with a
 # last round of half tiles (one of them past the last channel)
-SHAPES = [(1, 16, 16), (65, 144, 48), (63, 1056, 1536), (64, 4096, 64), (257, 4240, 1520), (17, 8960, 1536),
+SHAPES = [(1, 16, 16), (65, 144, 48), (63, 1056, 1536), (64, 4096, 64), (33, 4224, 192), (257, 4240, 1520), (17, 8960, 1536),
           (1000, 272, 2048), (1509, 1536, 1536), (2305, 128, 2320), (6032, 256, 1536), (2048, 400, 8192),
           (3105, 256, 8976), (6032, 1536, 8960), (8200, 400, 2144)]
 
