@@ -419,14 +419,12 @@ DIM, FFN = 1536, 8960       # the DiT's model and feed-forward widths
 def fp8_linear_calls(dev, steps=30):
     """The DiT's FP8 linears at the chunk shape (6032 tokens): q/k/v/o (1536 -> 1536) and the two feed-forward
     layers (1536 -> 8960, 8960 -> 1536), without gradients. Per call: the activation quantisation (lbw_quant_rows_fp8)
-    and the rowwise-scaled FP8 GEMM with the bias (lbw_gemm_fp8_rows; the tuned-solution table of the library GEMM is
-    read for the second timing, `ms`, and changes nothing on this path). Flops 2 M K N against 5.0 PFLOP/s dense fp8.
+    and the rowwise-scaled FP8 GEMM with the bias (lbw_gemm_fp8_rows). Flops 2 M K N against 5.0 PFLOP/s dense fp8.
     act_quant_call_ms times the quantisation call alone from Python; at ~6-9 us of kernel time it is bound by the
     launch path, so it is an upper bound on the kernel."""
     import torch
     from lingbot_world_v2_realtime_amd import kernels
-    import torch.cuda.tunable as tunable
-    from lingbot_world_v2_realtime_amd.layers.linear import FP8Linear, use_tuned_gemms
+    from lingbot_world_v2_realtime_amd.layers.linear import FP8Linear
     out = {}
     stream = torch.cuda.current_stream(dev)
     for name, (k, n) in (("proj_1536x1536", (DIM, DIM)), ("ffn_up_1536x8960", (DIM, FFN)),
@@ -434,21 +432,14 @@ def fp8_linear_calls(dev, steps=30):
         lin = torch.nn.Linear(k, n).to(torch.bfloat16).to(dev).requires_grad_(False)
         f = FP8Linear(lin)
         x = torch.randn(1, LQ, k, device=dev).to(torch.bfloat16)
-        times = {}
-        for mode in ("default", "table"):
-            table = use_tuned_gemms() if mode == "table" else False
-            for _ in range(3):
-                f(x)
-            torch.cuda.synchronize()
-            times[mode] = _timed(lambda: f(x), steps, stream)
-            if mode == "table":
-                tunable.enable(False)
-        ms = times["table"] if table else times["default"]
+        for _ in range(3):
+            f(x)
+        torch.cuda.synchronize()
+        ms = _timed(lambda: f(x), steps, stream)
         q_ms = _timed(lambda: kernels.quant_rows_fp8(x.view(LQ, k)), steps, stream)
         flops = 2.0 * LQ * k * n
         tf = flops / (ms * 1e-3) / 1e12
-        out[name] = {"ms": round(ms, 4), "default_solution_ms": round(times["default"], 4), "gemm_table": table,
-                     "act_quant_call_ms": round(q_ms, 4), "TFLOP/s": round(tf, 1),
+        out[name] = {"ms": round(ms, 4), "act_quant_call_ms": round(q_ms, 4), "TFLOP/s": round(tf, 1),
                      "frac_fp8_peak": round(tf / FP8_PEAK_TFLOPS, 4)}
     # the feed-forward block's GELU + down projection: torch's GELU then the FP8 linear (two passes over the
     # 6032 x 8960 activation), against the GELU fused into the activation quantisation (FP8Linear gelu_input,
@@ -456,7 +447,6 @@ def fp8_linear_calls(dev, steps=30):
     lin = torch.nn.Linear(FFN, DIM).to(torch.bfloat16).to(dev).requires_grad_(False)
     plain, fused = FP8Linear(lin), FP8Linear(lin, gelu_input=True)
     h = torch.randn(1, LQ, FFN, device=dev).to(torch.bfloat16)
-    table = use_tuned_gemms()
     unfused_fn = lambda: plain(torch.nn.functional.gelu(h, approximate="tanh"))   # noqa: E731
     fused_fn = lambda: fused(h)                                                   # noqa: E731
     for fn in (unfused_fn, fused_fn):
@@ -466,9 +456,8 @@ def fp8_linear_calls(dev, steps=30):
     t_unfused = _timed(unfused_fn, steps, stream)
     t_fused = _timed(fused_fn, steps, stream)
     t_gq = _timed(lambda: kernels.quant_rows_fp8_gelu(h.view(LQ, FFN)), steps, stream)
-    tunable.enable(False)
     out["ffn_gelu_down_8960x1536"] = {"ms": round(t_fused, 4), "unfused_ms": round(t_unfused, 4),
-                                      "gelu_act_quant_call_ms": round(t_gq, 4), "gemm_table": table}
+                                      "gelu_act_quant_call_ms": round(t_gq, 4)}
     # the MXFP8 mode (per-32 E8M0 scales) at the projection shape
     from lingbot_world_v2_realtime_amd.layers.linear import MXFP8Linear
     lin = torch.nn.Linear(DIM, DIM).to(torch.bfloat16).to(dev).requires_grad_(False)

@@ -547,6 +547,10 @@ static void gemm_launch(GemmArgs& a, hipStream_t stream, int64_t first = 0, int6
 // rounds x (stages x time of a stage + fixed part) as fitted to these figures. The MX form of 256 x 256 does not fit
 // the registers beside its scales (29.3 us against 29.3 for 192 x 192 at 1508 x 1536 x 8960, 114 against 102 at 6032
 // tokens), so MX stops at 192 x 192.
+// Behind the library GEMM by itself where tiles are few: 8960 x 1536 takes 14.3-14.8 against 10.4-10.8 us at 16 to 128
+// tokens (14.6 against 13.5 at 64), 16.1 against 15.3 at 257, 27.5 against 26.1-26.7 at 700 and 1024; 1536 x 1536 and
+// 2048 x 1024 are 0.5-0.9 us behind at up to 128 (24 tiles of long K on 256 CUs: K is not split over workgroups). A call
+// from Python is shorter all the same, 20 us of host work against 40; in a captured graph these shapes lose.
 // A last round of at most 128 such tiles goes out as half tiles in a launch of its own, which takes about half a
 // round (a half past the last channel is passed over): feed-forward at 6032 tokens 197.8 -> 192.0 us. (In the same launch,
 // after the whole tiles, the second tile body cost 28 spilled registers and 7 us.)

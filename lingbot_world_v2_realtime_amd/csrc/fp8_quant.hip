@@ -89,6 +89,7 @@ __device__ __forceinline__ uint32_t abs_bits(float x) { return __float_as_uint(x
 // thread's chunks in whatever form amax_bits() takes to abs_bits.
 template <bool GELU, typename T>
 struct Chunk {
+  static_assert(!GELU, "GELU has a form for bf16 rows only");
   float f[8];
   __device__ __forceinline__ void load(const T* p, uint32_t& amax) {
     Row8<T>::load(p, f);

@@ -22,7 +22,8 @@ from .. import kernels
 __all__ = ["FP8Linear", "MXFP8Linear", "convert_to_fp8", "fp8_eligible", "use_tuned_gemms", "tune_gemms",
            "GEMM_TABLE"]
 
-# hipBLASLt solutions for the DiT's rowwise FP8 GEMMs at the chunk shape (6032 tokens), as a TunableOp results file:
+# hipBLASLt solutions for the DiT's rowwise FP8 GEMMs at the chunk shape (6032 tokens), as a TunableOp results file (what
+# torch._scaled_mm takes; lbw_gemm_fp8_rows does not look at it):
 # a key per (layout, N, M, K, leading dims, rowwise scales, bias type), the solution, its measured time, and the
 # torch / HIP / hipBLASLt versions and GPU it holds for. Only the 8960 -> 1536 feed-forward projection is listed:
 # its tuned solution runs in 74-76 us against 96-97 us for the default pick; for 1536 -> 1536 and 1536 -> 8960 the
