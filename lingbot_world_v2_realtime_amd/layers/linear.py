@@ -161,22 +161,24 @@ class MXFP8Linear(torch.nn.Module):
         w8, w_scale, bias = self.w8, self.w_scale, self.bias
         if bias is not None:
             bias = bias.to(torch.bfloat16)
-        if not _plain(w8, w_scale) or not w8.is_contiguous():
+        plain = _plain(w8, w_scale, bias)
+        if not (plain or _plain(w8, w_scale)) or not w8.is_contiguous():
             m = x2.shape[0]
             x8, xs = kernels.quant_mx_fp8(x2.contiguous(), _pad(m, MX_ROWS))
             y = torch._scaled_mm(x8, w8.t(), scale_a=xs, scale_b=w_scale, out_dtype=torch.bfloat16)[:m]
             return self._add_bias(y, bias, shape)
         # the weights' scales go into the GEMM's order on every call: a kept copy would not follow writes to w_scale
         x8, xs, ws = kernels.quant_mx_fp8(x2.contiguous(), transposed=True, w_scale=w_scale)
-        fused = bias is not None and _plain(bias) and bias.shape == w8.shape[:1] == (self.out_features,)
+        fused = plain and bias is not None and bias.shape == w8.shape[:1] == (self.out_features,)
         y = kernels.gemm_fp8_mx(x8, xs, w8, ws, bias if fused else None)
         return self._add_bias(y, None if fused else bias, shape)
 
     def _add_bias(self, y, bias, shape):
-        y = y[:, :self.out_features]
+        if y.shape[1] != self.out_features:
+            y = y[:, :self.out_features]
         if bias is not None:
             y = y + bias
-        return y.reshape(*shape[:-1], self.out_features)
+        return y if len(shape) == 2 else y.reshape(*shape[:-1], self.out_features)
 
 
 def fp8_eligible(lin, mx=False):
